@@ -10,12 +10,15 @@
 //      (I, r) = min(C, C (x) D_rr) for all I, J != r: one launch;
 //   3. every other tile (I, J) = min(C, D_Ir (x) D_rJ): one launch.
 // Phases 2 and 3 reuse the register-blocked min-plus tile (minplus_tile.h)
-// with T x T tiles.  T = 128 halves the number of rounds and, with 8 x 8
+// with T x T tiles; phase 3 of T = 128 runs its additions on the matrix cores
+// (mfma_tile.h).  T = 128 halves the number of rounds and, with 8 x 8
 // cells per lane, the LDS bytes per update (phase 3 is bound by LDS reads
 // at 4 x 4 cells); T = 64 gives 4x more tiles per launch and a cheap
 // diagonal phase.  128 is the default for large n, 64 below (launch_fw).
+#include <type_traits>
+
 #include "common.h"
-#include "minplus_tile.h"
+#include "mfma_tile.h"
 
 namespace fapk {
 
@@ -191,7 +194,7 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(8)))
 template <int TM>
 __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void fw_rest_kernel(
     int32_t *d, int n, int64_t ld, int r, int nb, int flags, int mode, int fuse) {
-  using Tile = MpTile<TM, TM>;
+  using Tile = typename std::conditional<TM == 8, MxBig, MpTile<TM, TM>>::type;
   constexpr int T = Tile::BM;
   constexpr int LDS_WORDS = BLK_LDS_WORDS > Tile::LDS_WORDS ? BLK_LDS_WORDS : Tile::LDS_WORDS;
   __shared__ __attribute__((aligned(16))) int32_t lds[LDS_WORDS];

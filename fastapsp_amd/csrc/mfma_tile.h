@@ -1,0 +1,302 @@
+// mfma_tile.h -- min-plus tile whose additions run on the matrix cores.
+//
+// A min-plus update is an addition and a minimum.  On the VALU alone the pair
+// costs 1.5 instructions (v_add_u32 and half a v_min3_i32), and the tile of
+// minplus_tile.h runs at that limit.  Here the additions are an outer sum on
+// the matrix cores: with operands split in two f16 digits,
+//   (a.lo, a.hi, w0, w1) . (w0, w1, b.lo, b.hi) = w0 (a.lo + b.lo) + w1 (a.hi + b.hi),
+// one v_mfma_f32_32x32x4_2b_f16 (K = 4, two blocks: k and k + 1) makes
+// 2 x 32 x 32 sums a + b, and the VALU only folds them: one v_min3_i32 per
+// two updates.
+//
+// Exactness.  A digit is an 11-bit integer x stored as the f16 with bits x,
+// which is x 2^-24 exactly (subnormal below 1024, the first binade above; the
+// matrix cores of this target keep f16 subnormals).  With w0 = 1, w1 = 2048
+// the result is (a + b) 2^-24 for values below 2^22: every product and sum is
+// an integer below 2^24 times 2^-24, exact in float; sums are not negative, so
+// the minimum is taken on the floats' bits, as integers.  Operands are stored
+// plus one, so that INF = 2^30 - 1 becomes the single bit 30, which lands in
+// the exponent of the high digit: it reads as 2.0, the sum as at least 4096,
+// above every finite one.  A value that is neither below 2^22 - 1 nor INF or
+// above (bits 22..29 or the sign after the increment) raises a flag while it
+// is staged and the workgroup computes its tile again with integer additions
+// (MpTile): results are the same for all inputs.
+//
+// What bounds it: the VALU port, 16 v_min3_i32 and one MFMA issue for 2048
+// sums.  Measured in registers and LDS alone (4 waves per SIMD): 102 TOP/s at
+// 2 ops per update against 70.3 of add, add, min3 (MFMA alone 149, v_min3
+// alone 137; the clock falls to 2.1 GHz with both units busy).  Kernels on the
+// 128 x 128 tile, integer tile before: the 8192^3 product 16.5 -> 11.15 ms
+// (98.6 TOP/s), 909 x 262144 x 115 0.888 -> 0.689 ms, the n = 8192 closure
+// 19.0 -> 15.1 ms.  Every product of more than 16 rows takes it: short k and
+// edge tiles gain too, and values past the digits cost the first chunk.
+#ifndef FAP_MFMA_TILE_H_
+#define FAP_MFMA_TILE_H_
+
+#include "minplus_tile.h"
+
+namespace fapk {
+
+typedef _Float16 mx_half4 __attribute__((ext_vector_type(4)));
+typedef float mx_f32x32 __attribute__((ext_vector_type(32)));
+typedef int mx_int2 __attribute__((ext_vector_type(2)));
+
+constexpr int MX_BK = 8;                            // k per staged chunk
+constexpr uint32_t MX_WEIGHTS = 0x68003C00u;        // f16 {1.0, 2048.0}
+constexpr uint32_t MX_BAD = 0xBFC00000u;            // bits of v + 1 that leave the digits
+// v + 1 as two 11-bit f16 digits (high digit in the high half); bit 30, set
+// for INF alone among valid values, stays in place.
+__device__ __forceinline__ uint32_t mx_digits(uint32_t w) {
+  return __umul24((w >> 11) & 0x7FFu, 65536u - 2048u) + w;
+}
+
+typedef __attribute__((address_space(3))) int32_t *mx_lds_ptr;
+typedef __attribute__((address_space(1))) const int32_t *mx_in_ptr;
+typedef __attribute__((address_space(1))) int32_t *mx_out_ptr;
+
+// The same tile with integer additions, as a function of its own: inlined,
+// its registers and the matrix tile's accumulators would be live together
+// (both spilled: 8192^3 on values that the digits do not hold took 42.8 ms;
+// 19.3 ms this way, 18.8 ms on the integer tile alone).
+template <int NI, int NJ>
+__device__ __attribute__((noinline)) void int_tile(mx_in_ptr A, int64_t lda, mx_in_ptr B,
+                                                   int64_t ldb, mx_out_ptr C, int64_t ldc,
+                                                   int m_valid, int n_valid, int K,
+                                                   bool accumulate, int flags, mx_lds_ptr lds) {
+  __syncthreads();
+  MpTile<4 * NI, 4 * NJ>::run((const int32_t *)A, lda, (const int32_t *)B, ldb, (int32_t *)C, ldc,
+                              m_valid, n_valid, K, accumulate, flags, (int32_t *)lds);
+}
+
+// The tile: (64 NI) x (64 NJ) outputs by 256 threads, a wave (32 NI) x (32 NJ)
+// as NI x NJ MFMA blocks.  Element (k, row) of A and (k, column) of B are
+// 8 bytes in LDS, {digits, weights} and {weights, digits}; a fragment is one
+// ds_read_b64, lanes 0..31 at k and 32..63 at k + 1.  Lane l holds column
+// (l & 31) of a block and rows 8 (r / 4) + 4 (l / 32) + r % 4, r < 16.
+// k is staged in chunks of 8 in two LDS buffers (one barrier per chunk); the
+// next chunk's global loads are in flight while the current one is computed.
+// 128 VGPRs for 2 x 2 blocks: 64 accumulators, 32 sums, 8 staged words.
+template <int NI, int NJ>
+struct MxTile {
+  static constexpr int BM = 64 * NI, BN = 64 * NJ;
+  static constexpr int LDA = BM + 1, LDB = BN + 1;  // elements per k row
+  static constexpr int EA = 2 * NI, EB = 2 * NJ;    // staged words per thread
+  static constexpr int A_TPR = MX_BK / EA;          // threads per A row when staging
+  static constexpr int B_OFF = 2 * MX_BK * LDA;     // words from A to B of a buffer
+  static constexpr int BUF = 2 * MX_BK * (LDA + LDB);
+  static constexpr int FLAG = 2 * BUF;
+  static constexpr int LDS_WORDS = FLAG + 4;
+
+  template <int E>
+  __device__ static __forceinline__ void load_vec(const int32_t *base, uint32_t off, int v[E]) {
+    typedef int vec __attribute__((ext_vector_type(E), aligned(4)));
+    const vec x = *reinterpret_cast<const vec *>(reinterpret_cast<const char *>(base) + off);
+#pragma unroll
+    for (int i = 0; i < E; i++) v[i] = x[i];
+  }
+
+  // What the staging below asks of an operand: a full chunk and vector of
+  // columns, and byte offsets inside a chunk that fit 32 bits.
+  __device__ static __forceinline__ bool fits(int64_t lda, int64_t ldb, int n_valid, int K) {
+    return K >= MX_BK && n_valid >= EB && lda < (1 << 22) && ldb < (1 << 26);
+  }
+
+  // Where this thread's words of a chunk are: A row t / A_TPR, k
+  // (t % A_TPR) * EA ..; B k row t / 32, columns (t % 32) * EB ...  Rows past
+  // m_valid repeat the last one, columns past n_valid the last EB valid ones
+  // (at their own place): neither reaches a stored output.
+  struct Stage {
+    uint32_t a_off, b_off;  // bytes from the chunk's corner
+    int a_lds, b_lds;       // words from the buffer's start
+    __device__ __forceinline__ Stage(int64_t lda, int64_t ldb, int m_valid, int n_valid) {
+      const int t = threadIdx.x;
+      const int col = imin((t & 31) * EB, n_valid - EB);
+      a_off = 4u * ((uint32_t)imin(t / A_TPR, m_valid - 1) * (uint32_t)lda +
+                    (uint32_t)((t % A_TPR) * EA));
+      b_off = 4u * ((uint32_t)(t >> 5) * (uint32_t)ldb + (uint32_t)col);
+      a_lds = 2 * ((t % A_TPR) * EA * LDA + t / A_TPR);
+      b_lds = B_OFF + 2 * ((t >> 5) * LDB + col) + 1;
+    }
+  };
+
+  // Writes the digits of a loaded chunk to `buf`; returns the bits seen
+  // outside them.
+  __device__ static __forceinline__ uint32_t store_chunk(int32_t *buf, const Stage &st,
+                                                         const int ra[EA], const int rb[EB]) {
+    uint32_t seen = 0;
+    int32_t *pa = buf + st.a_lds;
+#pragma unroll
+    for (int i = 0; i < EA; i++) {
+      const uint32_t w = (uint32_t)ra[i] + 1u;
+      seen |= w;
+      pa[2 * i * LDA] = (int32_t)mx_digits(w);
+    }
+    int32_t *pb = buf + st.b_lds;
+#pragma unroll
+    for (int i = 0; i < EB; i++) {
+      const uint32_t w = (uint32_t)rb[i] + 1u;
+      seen |= w;
+      pb[2 * i] = (int32_t)mx_digits(w);
+    }
+    return seen & MX_BAD;
+  }
+
+  // The constant halves of both buffers' elements, and the flags: once.
+  __device__ static __forceinline__ void init_lds(int32_t *lds) {
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+      for (int i = threadIdx.x; i < MX_BK * LDA; i += MP_THREADS)
+        lds[b * BUF + 2 * i + 1] = (int32_t)MX_WEIGHTS;
+      for (int i = threadIdx.x; i < MX_BK * LDB; i += MP_THREADS)
+        lds[b * BUF + B_OFF + 2 * i] = (int32_t)MX_WEIGHTS;
+    }
+    if (threadIdx.x < 2) lds[FLAG + threadIdx.x] = 0;
+  }
+
+  // acc = min(acc, A (x) B) over the staged chunk's k from kbeg (even) on, as
+  // float bits.  A block of 16 minima follows each MFMA; the other waves of
+  // the SIMD issue while its result is in flight.
+  __device__ static __forceinline__ void compute(const int32_t *buf, int kbeg,
+                                                 int acc[NI][NJ][16]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const mx_int2 *pa = reinterpret_cast<const mx_int2 *>(buf) + (kbeg + (lane >> 5)) * LDA +
+                        (wave >> 1) * (32 * NI) + (lane & 31);
+    const mx_int2 *pb = reinterpret_cast<const mx_int2 *>(buf + B_OFF) + (kbeg + (lane >> 5)) * LDB +
+                        (wave & 1) * (32 * NJ) + (lane & 31);
+    mx_f32x32 zero;
+#pragma unroll
+    for (int r = 0; r < 32; r++) zero[r] = 0.0f;
+#pragma unroll 1
+    for (int kk = kbeg; kk < MX_BK; kk += 2) {
+      mx_half4 a[NI], b[NJ];
+#pragma unroll
+      for (int i = 0; i < NI; i++) a[i] = __builtin_bit_cast(mx_half4, pa[32 * i]);
+#pragma unroll
+      for (int j = 0; j < NJ; j++) b[j] = __builtin_bit_cast(mx_half4, pb[32 * j]);
+      pa += 2 * LDA;
+      pb += 2 * LDB;
+#pragma unroll
+      for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+          const mx_f32x32 d = __builtin_amdgcn_mfma_f32_32x32x4f16(a[i], b[j], zero, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 16; r++)
+            acc[i][j][r] = imin(acc[i][j][r], imin(__float_as_int(d[r]), __float_as_int(d[16 + r])));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+  }
+
+  // The value of an accumulator: the sum less both operands' + 1.  The
+  // instruction saturates (a C++ cast need not), so every sum with an INF in
+  // it comes out as INF.
+  __device__ static __forceinline__ int value(int bits) {
+    int v;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(v) : "v"(fmaf(__int_as_float(bits), 16777216.0f, -2.0f)));
+    return imin(v, kInf);
+  }
+
+  // Row of a block held in accumulator r by lanes 0..31 (4 more above).
+  __device__ static constexpr int acc_row(int r) { return 8 * (r >> 2) + (r & 3); }
+
+  // The k loop: staging pipelined with compute.  The last chunk ends at K
+  // and skips (pairwise) the k that the one before it has taken.  Returns
+  // nonzero (the same for every thread) when a value did not fit its digits.
+  // Two flags, by chunk parity: one is read after the barrier that follows
+  // its last possible write, while a faster thread may already be writing the
+  // other.
+  __device__ static __forceinline__ int product(const int32_t *A, int64_t lda, const int32_t *B,
+                                                int64_t ldb, int m_valid, int n_valid, int K,
+                                                int32_t *lds, int acc[NI][NJ][16]) {
+    int ra[EA], rb[EB];
+    const Stage st(lda, ldb, m_valid, n_valid);
+    load_vec<EA>(A, st.a_off, ra);
+    load_vec<EB>(B, st.b_off, rb);
+    init_lds(lds);
+    __syncthreads();  // the flags are cleared
+    if (store_chunk(lds, st, ra, rb)) lds[FLAG] = 1;
+    __syncthreads();
+    int kbeg = 0, par = 0;
+    for (int k0 = MX_BK;; k0 += MX_BK) {
+      const bool more = k0 < K;
+      const int kc = imin(k0, K - MX_BK);  // start of the next chunk
+      if (more) {
+        load_vec<EA>(A + kc, st.a_off, ra);
+        load_vec<EB>(B + (int64_t)kc * ldb, st.b_off, rb);
+      }
+      const int bad = __builtin_amdgcn_readfirstlane(lds[FLAG + par]);
+      if (bad) return 1;
+      compute(lds + par * BUF, kbeg, acc);
+      if (!more) return 0;
+      par ^= 1;
+      kbeg = (k0 - kc) & ~1;
+      if (store_chunk(lds + par * BUF, st, ra, rb)) lds[FLAG + par] = 1;
+      __syncthreads();
+    }
+  }
+
+  // Compute the tile, arguments as MpTile::run (m_valid, n_valid >= 1).  C
+  // may alias A or B: every operand is read before the epilogue writes (the
+  // last chunk's loads end before its barrier).
+  __device__ static __forceinline__ void run(const int32_t *A, int64_t lda, const int32_t *B,
+                                             int64_t ldb, int32_t *C, int64_t ldc, int m_valid,
+                                             int n_valid, int K, bool accumulate, int flags,
+                                             int32_t *lds) {
+    int acc[NI][NJ][16];
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+#pragma unroll
+      for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][j][r] = 0x7F800000;  // above every sum: INF
+    if (!fits(lda, ldb, n_valid, K) || product(A, lda, B, ldb, m_valid, n_valid, K, lds, acc)) {
+      int_tile<NI, NJ>((mx_in_ptr)A, lda, (mx_in_ptr)B, ldb, (mx_out_ptr)C, ldc, m_valid, n_valid,
+                       K, accumulate, flags, (mx_lds_ptr)lds);
+      return;
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int row0 = (wave >> 1) * (32 * NI) + (lane >> 5) * 4;
+    const int col0 = (wave & 1) * (32 * NJ) + (lane & 31);
+    const bool full = m_valid == BM && n_valid == BN;
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      int32_t *c = C + (int64_t)(row0 + 32 * i) * ldc + col0;
+      if (full) {
+        // the C words of a row of blocks are all loaded before any is
+        // stored: the compiler must assume that a store changes later loads
+        int o[NJ][16];
+        if (accumulate) {
+#pragma unroll
+          for (int r = 0; r < 16; r++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) o[j][r] = c[(int64_t)acc_row(r) * ldc + 32 * j];
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+#pragma unroll
+          for (int j = 0; j < NJ; j++) {
+            const int v = value(acc[i][j][r]);
+            c[(int64_t)acc_row(r) * ldc + 32 * j] = accumulate ? imin(v, o[j][r]) : v;
+          }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+#pragma unroll
+          for (int j = 0; j < NJ; j++)
+            if (row0 + 32 * i + acc_row(r) < m_valid && col0 + 32 * j < n_valid) {
+              const int v = value(acc[i][j][r]);
+              int32_t *p = c + (int64_t)acc_row(r) * ldc + 32 * j;
+              *p = accumulate ? imin(v, *p) : v;
+            }
+      }
+    }
+  }
+};
+
+using MxBig = MxTile<2, 2>;    // 128 x 128
+using MxSmall = MxTile<1, 1>;  // 64 x 64
+
+}  // namespace fapk
+
+#endif  // FAP_MFMA_TILE_H_

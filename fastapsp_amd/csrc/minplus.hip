@@ -1,11 +1,11 @@
-// minplus.hip -- min-plus product C = min(base, A (x) B) on the VALU.
+// minplus.hip -- min-plus product C = min(base, A (x) B).
 //
 // Replaces the reference's stage-3 operator (min_plus_path_advanced,
 // fap/kernel/minplus.h:78-89; CPU semantics :51-65: every output starts at
 // INF and takes the strict minimum over k).  One 128 x 128 tile per
-// workgroup, see minplus_tile.h for the register/LDS layout.
+// workgroup, additions on the matrix cores (mfma_tile.h).
 #include "common.h"
-#include "minplus_tile.h"
+#include "mfma_tile.h"
 
 namespace fapk {
 
@@ -28,12 +28,12 @@ __device__ __forceinline__ void gemm_tile_coords(int bid, int tiles_m, int tiles
 __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void minplus_gemm_kernel(
     const int32_t *A, int64_t lda, const int32_t *B, int64_t ldb, int32_t *C, int64_t ldc,
     int M, int N, int K, int accumulate, int flags, int tiles_m, int tiles_n) {
-  __shared__ __attribute__((aligned(16))) int32_t lds[MpBig::LDS_WORDS];
+  __shared__ __attribute__((aligned(16))) int32_t lds[MxBig::LDS_WORDS];
   int tm, tn;
   gemm_tile_coords(blockIdx.x, tiles_m, tiles_n, &tm, &tn);
   const int m0 = tm * MP_BM, n0 = tn * MP_BN;
-  MpBig::run(A + (int64_t)m0 * lda, lda, B + n0, ldb, C + (int64_t)m0 * ldc + n0, ldc,
-             imin(MP_BM, M - m0), imin(MP_BN, N - n0), K, accumulate != 0, flags, lds);
+  MxBig::run(A + (int64_t)m0 * lda, lda, B + n0, ldb, C + (int64_t)m0 * ldc + n0, ldc,
+              imin(MP_BM, M - m0), imin(MP_BN, N - n0), K, accumulate != 0, flags, lds);
 }
 
 // The last rows of a product whose row count leaves at most 64 rows past

@@ -44,40 +44,6 @@
 
 namespace fapk {
 
-// Launches of diagonal tasks only: one 1024-thread workgroup per task, a
-// thread per 1 x 4 strip (lds_fw64, as the dense diagonal kernel), about
-// twice as fast per block as the 256-thread closure.
-__global__ __launch_bounds__(1024) void fw_diag_batch_kernel(const BatchJob *__restrict__ jobs,
-                                                            const BatchSeg *__restrict__ segs,
-                                                            int nseg, int ntasks) {
-  __shared__ __attribute__((aligned(16))) int32_t D[BLK_LDS_WORDS];
-  const int t = threadIdx.x;
-  for (int ti = blockIdx.x; ti < ntasks; ti += gridDim.x) {
-    int lo = 0, hi = nseg - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (segs[mid].first <= ti) lo = mid;
-      else hi = mid - 1;
-    }
-    const BatchSeg sg = segs[lo];
-    const BatchJob job = jobs[sg.job];
-    const int base = (sg.kind_r >> 3) * BT;
-    const int kb = imin(BT, job.n - base);
-    int32_t *blk = job.mat + (int64_t)base * job.ld + base;
-    for (int idx = t; idx < 64 * 64; idx += 1024) {
-      const int i = idx >> 6, j = idx & 63;
-      D[i * BLK_LD + j] = (i < kb && j < kb) ? blk[(int64_t)i * job.ld + j] : kInf;
-    }
-    __syncthreads();
-    lds_fw64<BLK_LD>(D, 0, kb);
-    for (int idx = t; idx < 64 * 64; idx += 1024) {
-      const int i = idx >> 6, j = idx & 63;
-      if (i < kb && j < kb) blk[(int64_t)i * job.ld + j] = D[i * BLK_LD + j];
-    }
-    __syncthreads();  // the LDS tile is reused by the next task
-  }
-}
-
 // The segment holding task ti: segments tile [0, ntasks) in order.
 template <typename Seg>
 __device__ __forceinline__ int find_seg(const Seg *__restrict__ segs, int nseg, int ti) {
@@ -88,6 +54,20 @@ __device__ __forceinline__ int find_seg(const Seg *__restrict__ segs, int nseg, 
     else hi = mid - 1;
   }
   return lo;
+}
+
+// Launches of diagonal tasks only: a workgroup per block, held in registers
+// (close64).
+constexpr int DIAG_THREADS = 512;
+__global__ __launch_bounds__(DIAG_THREADS) void fw_diag_batch_kernel(
+    const BatchJob *__restrict__ jobs, const BatchSeg *__restrict__ segs, int nseg, int ntasks) {
+  __shared__ __attribute__((aligned(16))) int32_t buf[CLOSE64_WORDS];
+  for (int ti = blockIdx.x; ti < ntasks; ti += gridDim.x) {
+    const BatchSeg sg = segs[find_seg(segs, nseg, ti)];
+    const BatchJob job = jobs[sg.job];
+    const int base = (sg.kind_r >> 3) * BT;
+    close_block64<2>(job.mat + (int64_t)base * job.ld + base, job.ld, imin(BT, job.n - base), buf);
+  }
 }
 
 // Task idx of a panel, single-pivot (rest and cross kinds) or pair-pass
@@ -197,7 +177,7 @@ __global__ void xcc_probe_kernel(int32_t *mask) {
 __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void fw_queue_kernel(
     const BatchJob *__restrict__ jobs, const int32_t *__restrict__ qinfo,
     const int4 *__restrict__ all_rec, int32_t *ctrl, int32_t *done, int64_t limit) {
-  constexpr int W = BLK_LDS_WORDS > MpSmall::LDS_WORDS ? BLK_LDS_WORDS : MpSmall::LDS_WORDS;
+  constexpr int W = CLOSE64_WORDS > MpSmall::LDS_WORDS ? CLOSE64_WORDS : MpSmall::LDS_WORDS;
   __shared__ __attribute__((aligned(16))) int32_t lds[W];
   __shared__ int32_t s_next, s_go;
   const int t = threadIdx.x;
@@ -245,7 +225,7 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(6)))
     const int kind = tr.y & 7, r = tr.y >> 3;
     if (kind == TASK_DIAG) {
       const int base = r * BT;
-      close_block64(job.mat + (int64_t)base * job.ld + base, job.ld, imin(BT, job.n - base), lds);
+      close_block64<4>(job.mat + (int64_t)base * job.ld + base, job.ld, imin(BT, job.n - base), lds);
     } else {
       batch_tile_task(job, kind, r, tr.z, lds);
     }
@@ -575,8 +555,8 @@ int launch_fw_batch(fap_ctx *ctx, const FwBatchDesc &desc, const fapk::BatchJob 
     const dim3 grid(std::min(cnt, cap)), block(fapk::MP_THREADS);
     const fapk::BatchSeg *sg = d_segs + desc.seg_off[p];
     if (kind == fapk::TASK_DIAG)
-      hipLaunchKernelGGL(fapk::fw_diag_batch_kernel, dim3(std::min(cnt, ctx->num_cus * 2)),
-                         dim3(1024), 0, s, d_jobs, sg, nseg, cnt);
+      hipLaunchKernelGGL(fapk::fw_diag_batch_kernel, dim3(std::min(cnt, ctx->num_cus * 4)),
+                         dim3(fapk::DIAG_THREADS), 0, s, d_jobs, sg, nseg, cnt);
     else if (kind == fapk::TASK_PANEL)
       hipLaunchKernelGGL(fapk::fw_phase_kernel<fapk::TASK_PANEL>, grid, block, 0, s, d_jobs, sg,
                          nseg, cnt);

@@ -22,70 +22,128 @@
 
 namespace fapk {
 
-constexpr int FW_DIAG_THREADS = 1024;
+// Closure of a 128 x 128 diagonal block (kb <= 128 valid rows/columns) by
+// one workgroup of 1024 / NC threads: the blocked algorithm itself one level
+// down, its 64-blocks closed in registers and multiplied from LDS (Blk64).
+// The four blocks stay in registers throughout, so memory is read and
+// written once.  `lds` holds CLOSE128_WORDS.
+constexpr int CLOSE128_WORDS = 2 * T64_WORDS + CLOSE64_WORDS;
 
-// In-LDS helpers for the diagonal tile (1024 threads).  The tile lives in
-// D[T][T + 4] (rows 16-byte aligned); lds_fw64 (minplus_tile.h) closes a
-// 64 x 64 sub-block of it.
-
-// C = min(C, A (x) B) for 64 x 64 sub-blocks given by their corners
-// (row, col) in D, K = 64.  All reads happen before the barrier that
-// precedes the writes, so C may alias A or B.
-template <int LD>
-__device__ __forceinline__ void lds_mp64(int32_t *D, int ci, int cj, int ai, int ak, int bk,
-                                         int bj) {
-  const int t = threadIdx.x;
-  const int r = t >> 4, c0 = (t & 15) << 2;
-  int4 acc = *reinterpret_cast<const int4 *>(D + (ci + r) * LD + cj + c0);
-  const int32_t *arow = D + (ai + r) * LD + ak;
-#pragma unroll 4
-  for (int k = 0; k < 64; k += 2) {
-    const int2 a = *reinterpret_cast<const int2 *>(arow + k);
-    const int4 b0 = *reinterpret_cast<const int4 *>(D + (bk + k) * LD + bj + c0);
-    const int4 b1 = *reinterpret_cast<const int4 *>(D + (bk + k + 1) * LD + bj + c0);
-    acc.x = imin(acc.x, imin(a.x + b0.x, a.y + b1.x));
-    acc.y = imin(acc.y, imin(a.x + b0.y, a.y + b1.y));
-    acc.z = imin(acc.z, imin(a.x + b0.z, a.y + b1.z));
-    acc.w = imin(acc.w, imin(a.x + b0.w, a.y + b1.w));
+template <int NC>
+__device__ __forceinline__ void close_block128(int32_t *blk, int64_t ld, int kb, int32_t *lds) {
+  using B = Blk64<NC>;
+  int32_t *X = lds, *Y = lds + T64_WORDS, *buf = lds + 2 * T64_WORDS;
+  const int n0 = imin(64, kb), n1 = kb - 64;
+  int d00[4][NC], d01[4][NC], d10[4][NC], d11[4][NC];
+  int32_t *p01 = blk + 64, *p10 = blk + 64 * ld, *p11 = blk + 64 * ld + 64;
+  if (n1 <= 0) {
+    close_block64<NC>(blk, ld, n0, buf);
+    return;
   }
+  B::load(blk, ld, n0, n0, d00);
+  B::load(p01, ld, n0, n1, d01);
+  B::load(p10, ld, n1, n0, d10);
+  B::load(p11, ld, n1, n1, d11);
+  B::close(d00, n0, buf);
+  B::to_lds(X, d00);
+  B::to_lds(Y, d01);
   __syncthreads();
-  *reinterpret_cast<int4 *>(D + (ci + r) * LD + cj + c0) = acc;
+  B::product(X, Y, d01);  // D01 (+)= D00 D01
   __syncthreads();
+  B::to_lds(Y, d10);
+  __syncthreads();
+  B::product(Y, X, d10);  // D10 (+)= D10 D00
+  __syncthreads();
+  B::to_lds(X, d10);
+  B::to_lds(Y, d01);
+  __syncthreads();
+  B::product(X, Y, d11);  // D11 (+)= D10 D01
+  B::close(d11, n1, buf);
+  B::to_lds(X, d11);  // X's readers have passed a barrier of the closure
+  __syncthreads();
+  B::product(Y, X, d01);  // D01 (+)= D01 D11
+  __syncthreads();
+  B::to_lds(Y, d10);
+  __syncthreads();
+  B::product(X, Y, d10);  // D10 (+)= D11 D10
+  __syncthreads();
+  B::to_lds(X, d01);
+  B::to_lds(Y, d10);
+  __syncthreads();
+  B::product(X, Y, d00);  // D00 (+)= D01 D10
+  B::store(blk, ld, n0, n0, d00);
+  B::store(p01, ld, n0, n1, d01);
+  B::store(p10, ld, n1, n0, d10);
+  B::store(p11, ld, n1, n1, d11);
 }
 
-// Phase 1 for T = 64 (direct) or T = 128 (2 x 2 recursion on 64-blocks:
-// close D00; panels D01, D10; D11 += D10 D01; close D11; panels D10, D01;
-// D00 += D01 D10 -- the blocked algorithm itself, one level down, so most
-// of the work runs as min-plus products with two k per v_min3).
+// The closures as functions of their own, for kernels that reach them in one
+// workgroup: inlined, their cells would take registers from the tile loop.
 template <int T>
-__global__ __launch_bounds__(FW_DIAG_THREADS) void fw_diag_kernel(int32_t *d, int n,
-                                                                  int64_t ld, int r) {
-  constexpr int LD = T + 4;
-  __shared__ __attribute__((aligned(16))) int32_t D[T * LD];
+__device__ __attribute__((noinline)) void close_block_call(mx_out_ptr blk, int64_t ld, int kb,
+                                                           mx_lds_ptr lds) {
+  if (T == 128) close_block128<4>((int32_t *)blk, ld, kb, (int32_t *)lds);
+  else close_block64<4>((int32_t *)blk, ld, kb, (int32_t *)lds);
+}
+
+constexpr int FW_DIAG_THREADS = 512;  // workgroups alone on their CU: Blk64<2>
+
+// Phase 1: the diagonal tile (r, r) alone, one workgroup.
+template <int T>
+__global__ __launch_bounds__(FW_DIAG_THREADS) void fw_diag_kernel(int32_t *d, int n, int64_t ld,
+                                                                  int r) {
+  __shared__ __attribute__((aligned(16))) int32_t lds[T == 64 ? CLOSE64_WORDS : CLOSE128_WORDS];
   const int base = r * T;
   const int kb = imin(T, n - base);
   int32_t *blk = d + (int64_t)base * ld + base;
-  for (int idx = threadIdx.x; idx < T * T; idx += FW_DIAG_THREADS) {
-    const int i = idx / T, j = idx - (idx / T) * T;
-    D[i * LD + j] = (i < kb && j < kb) ? blk[(int64_t)i * ld + j] : kInf;
+  if (T == 64) close_block64<2>(blk, ld, kb, lds);
+  else close_block128<2>(blk, ld, kb, lds);
+}
+
+// One whole round of T = 64 in a launch, for matrices whose rounds are
+// latency and not work: the workgroup of tile (I, J) closes the pivot block
+// itself, forms the row panel tile it needs, B' = min(B, D* (x) B), and
+// updates C = min(C, A (x) B').  Sibling workgroups may already be writing
+// the closed pivot block and panels over the tiles read here; every value in
+// between is the length of a path through block r, no shorter than the
+// closed one, and min-plus with the closed block makes the same result of
+// both (D* D* = D*), so the bits do not depend on what was seen.
+__global__ __launch_bounds__(FW_DIAG_THREADS) void fw_round_kernel(int32_t *d, int n, int64_t ld,
+                                                                   int r, int nb) {
+  using Blk = Blk64<2>;
+  __shared__ __attribute__((aligned(16))) int32_t lds[3 * T64_WORDS + CLOSE64_WORDS];
+  int32_t *X = lds, *Y = lds + T64_WORDS, *Z = lds + 2 * T64_WORDS;
+  const int I = blockIdx.x / nb, J = blockIdx.x - I * nb;
+  const int base = r * 64;
+  const int kb = imin(64, n - base), rows = imin(64, n - I * 64), cols = imin(64, n - J * 64);
+  int32_t *tile = d + (int64_t)I * 64 * ld + (int64_t)J * 64;
+  int dd[4][2], a[4][2], b[4][2], c[4][2];
+  Blk::load(d + (int64_t)base * ld + base, ld, kb, kb, dd);
+  Blk::load(tile, ld, rows, cols, c);
+  if (I != r && J != r) {
+    Blk::load(d + (int64_t)base * ld + (int64_t)J * 64, ld, kb, cols, b);
+    Blk::load(d + (int64_t)I * 64 * ld + base, ld, rows, kb, a);
+  }
+  Blk::close(dd, kb, lds + 3 * T64_WORDS);
+  if (I == r && J == r) {
+    Blk::store(tile, ld, rows, cols, dd);
+    return;
+  }
+  Blk::to_lds(X, dd);
+  const bool rest = I != r && J != r;
+  if (rest) {
+    Blk::to_lds(Y, b);
+    Blk::to_lds(Z, a);
+    __syncthreads();
+    Blk::product(X, Y, b);
+    __syncthreads();
+    Blk::to_lds(Y, b);
+  } else {
+    Blk::to_lds(Y, c);
   }
   __syncthreads();
-  const int n0 = imin(64, kb);
-  lds_fw64<LD>(D, 0, n0);
-  if (T == 128 && kb > 64) {
-    const int n1 = kb - 64;
-    lds_mp64<LD>(D, 0, 64, 0, 0, 0, 64);    // D01 = min(D01, D00 D01)
-    lds_mp64<LD>(D, 64, 0, 64, 0, 0, 0);    // D10 = min(D10, D10 D00)
-    lds_mp64<LD>(D, 64, 64, 64, 0, 0, 64);  // D11 = min(D11, D10 D01)
-    lds_fw64<LD>(D, 64, n1);
-    lds_mp64<LD>(D, 64, 0, 64, 64, 64, 0);  // D10 = min(D10, D11 D10)
-    lds_mp64<LD>(D, 0, 64, 0, 64, 64, 64);  // D01 = min(D01, D01 D11)
-    lds_mp64<LD>(D, 0, 0, 0, 64, 64, 0);    // D00 = min(D00, D01 D10)
-  }
-  for (int idx = threadIdx.x; idx < T * T; idx += FW_DIAG_THREADS) {
-    const int i = idx / T, j = idx - (idx / T) * T;
-    if (i < kb && j < kb) blk[(int64_t)i * ld + j] = D[i * LD + j];
-  }
+  Blk::product(rest ? Z : I == r ? X : Y, J == r ? X : Y, c);
+  Blk::store(tile, ld, rows, cols, c);
 }
 
 // Phase 2: workgroups [0, nb-1) take row-panel tiles (r, J), the next nb-1
@@ -111,34 +169,6 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
     int32_t *c = d + (int64_t)I * T * ld + base;
     Tile::run(c, ld, diag, ld, c, ld, imin(T, n - I * T), kb, kb, true, flags, lds);
   }
-}
-
-// Closure of a 128 x 128 diagonal block (kb <= 128 valid rows/columns) by
-// one 256-thread workgroup, in global memory: the 2 x 2 recursion of
-// fw_diag_kernel<128> with each 64-block closed in LDS (close_block64) and
-// each 64 x 64 product done by the product tile (C may alias A or B: the
-// tile reads its operands before it writes).  `lds` holds BLK_LDS_WORDS.
-__device__ __forceinline__ void close_block128(int32_t *blk, int64_t ld, int kb, int flags,
-                                               int32_t *lds) {
-  const int n0 = imin(64, kb), n1 = kb - 64;
-  close_block64(blk, ld, n0, lds);
-  __syncthreads();
-  if (n1 <= 0) return;
-  int32_t *d00 = blk, *d01 = blk + 64, *d10 = blk + 64 * ld, *d11 = blk + 64 * ld + 64;
-  MpSmall::run(d00, ld, d01, ld, d01, ld, n0, n1, n0, true, flags, lds);  // D01 (+)= D00 D01
-  __syncthreads();
-  MpSmall::run(d10, ld, d00, ld, d10, ld, n1, n0, n0, true, flags, lds);  // D10 (+)= D10 D00
-  __syncthreads();
-  MpSmall::run(d10, ld, d01, ld, d11, ld, n1, n1, n0, true, flags, lds);  // D11 (+)= D10 D01
-  __syncthreads();
-  close_block64(d11, ld, n1, lds);
-  __syncthreads();
-  MpSmall::run(d11, ld, d10, ld, d10, ld, n1, n0, n1, true, flags, lds);  // D10 (+)= D11 D10
-  __syncthreads();
-  MpSmall::run(d01, ld, d11, ld, d01, ld, n0, n1, n1, true, flags, lds);  // D01 (+)= D01 D11
-  __syncthreads();
-  MpSmall::run(d01, ld, d10, ld, d00, ld, n0, n0, n1, true, flags, lds);  // D00 (+)= D01 D10
-  __syncthreads();
 }
 
 // Phase 2 for T = 128 in 64 x 64 pieces: each panel tile (r, J) or (I, r)
@@ -191,12 +221,13 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(8)))
 // it (in LDS for T = 64, by close_block128 for T = 128): the next round's
 // diagonal phase, done while the other tiles of this phase run, so that
 // round launches only its panels.
-template <int TM>
+template <int TM, bool fuse>
 __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void fw_rest_kernel(
-    int32_t *d, int n, int64_t ld, int r, int nb, int flags, int mode, int fuse) {
+    int32_t *d, int n, int64_t ld, int r, int nb, int flags, int mode) {
   using Tile = typename std::conditional<TM == 8, MxBig, MpTile<TM, TM>>::type;
   constexpr int T = Tile::BM;
-  constexpr int LDS_WORDS = BLK_LDS_WORDS > Tile::LDS_WORDS ? BLK_LDS_WORDS : Tile::LDS_WORDS;
+  constexpr int CLOSE_WORDS = TM == 4 ? CLOSE64_WORDS : CLOSE128_WORDS;
+  constexpr int LDS_WORDS = CLOSE_WORDS > Tile::LDS_WORDS ? CLOSE_WORDS : Tile::LDS_WORDS;
   __shared__ __attribute__((aligned(16))) int32_t lds[LDS_WORDS];
   int I, J;
   if (mode == 0) {
@@ -238,8 +269,7 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
   Tile::run(a, ld, b, ld, c, ld, imin(T, n - I * T), imin(T, n - J * T), kb, true, flags, lds);
   if (fuse && blockIdx.x == 0) {
     __syncthreads();  // the tile's writes above come before the closure reads it
-    if (TM == 4) close_block64(c, ld, imin(T, n - I * T), lds);
-    else close_block128(c, ld, imin(T, n - I * T), flags, lds);
+    close_block_call<T>((mx_out_ptr)c, ld, imin(T, n - I * T), (mx_lds_ptr)lds);
   }
 }
 
@@ -259,8 +289,8 @@ struct Fw {
   static int diag_panel(int32_t *d, int32_t n, int64_t ld, int r, int nb, int flags,
                         hipStream_t s, bool diag = true) {
     if (diag) {
-      hipLaunchKernelGGL(fapk::fw_diag_kernel<T>, dim3(1), dim3(fapk::FW_DIAG_THREADS), 0, s,
-                         d, n, ld, r);
+      hipLaunchKernelGGL(fapk::fw_diag_kernel<T>, dim3(1), dim3(fapk::FW_DIAG_THREADS), 0, s, d,
+                         n, ld, r);
       FAP_CHECK_LAUNCH();
     }
     if (nb > 1) {
@@ -280,8 +310,12 @@ struct Fw {
     const int tiles =
         mode == 0 ? (nb - 1) * (nb - 1) : mode == 1 ? 2 * nb - 3 : (nb - 2) * (nb - 2);
     if (tiles <= 0) return FAP_OK;
-    hipLaunchKernelGGL(fapk::fw_rest_kernel<TM>, dim3(tiles), dim3(fapk::MP_THREADS), 0, s, d,
-                       n, ld, r, nb, flags, mode, fuse);
+    if (fuse)
+      hipLaunchKernelGGL((fapk::fw_rest_kernel<TM, true>), dim3(tiles), dim3(fapk::MP_THREADS), 0,
+                         s, d, n, ld, r, nb, flags, mode);
+    else
+      hipLaunchKernelGGL((fapk::fw_rest_kernel<TM, false>), dim3(tiles), dim3(fapk::MP_THREADS), 0,
+                         s, d, n, ld, r, nb, flags, mode);
     FAP_CHECK_LAUNCH();
     return FAP_OK;
   }
@@ -326,6 +360,17 @@ struct Fw {
 
 }  // namespace
 
+// Rounds of T = 64 as single launches (fw_round_kernel).
+static int run_rounds(int32_t *d, int32_t n, int64_t ld, hipStream_t s) {
+  const int nb = (n + 63) / 64;
+  for (int r = 0; r < nb; r++) {
+    hipLaunchKernelGGL(fapk::fw_round_kernel, dim3(nb * nb), dim3(fapk::FW_DIAG_THREADS), 0, s,
+                       d, n, ld, r, nb);
+    FAP_CHECK_LAUNCH();
+  }
+  return FAP_OK;
+}
+
 // Block size and look-ahead: the context options if set, else the tune
 // cache, else 128 when phase 3 has at least 8 tiles of 128 per CU and 64
 // below, without look-ahead (fw_settings).  Measured on MI355X (closure
@@ -341,6 +386,13 @@ int launch_fw(fap_ctx *ctx, int32_t *d, int32_t n, int64_t ld, hipStream_t s) {
   bool lookahead;
   fw_settings(ctx, n, &tile, &lookahead);
   if (tile == 128) return Fw<8>::run(ctx, d, n, ld, lookahead, s);
+  // Up to 1.5 workgroups per CU a round in one launch wins although every
+  // workgroup closes the pivot block and makes its own panel tile (closure us,
+  // one / three launches a round: n = 97 44 / 66, 512 160 / 243, 1024 331 /
+  // 494, 1200 579 / 662; 1448 1021 / 829: two full workgroups per CU).
+  const int64_t nb = (n + 63) / 64;
+  if (!lookahead && 2 * nb * nb <= 3 * (int64_t)(ctx ? ctx->num_cus : 256))
+    return run_rounds(d, n, ld, s);
   return Fw<4>::run(ctx, d, n, ld, lookahead, s);
 }
 

@@ -263,68 +263,254 @@ struct MpTile {
 using MpBig = MpTile<8, 8>;    // 128 x 128
 using MpSmall = MpTile<4, 4>;  // 64 x 64
 
-// Floyd-Warshall closure of one diagonal block of up to 64 x 64 (kb valid
-// rows and columns; the rest read as INF) with 256 threads, in LDS (`D`
-// holds BLK_LDS_WORDS ints, row stride BLK_LD): thread t owns the 1 x 4
-// strips at rows (t >> 4) + 16q, q < 4, columns (t & 15) * 4.  Row k and
-// column k do not change during pivot k (the diagonal is >= 0), so every
-// thread updates in place; one barrier per pivot.
-// Closure of a 64 x 64 sub-block with 1024 threads: a thread owns the 1 x 4
-// strip at row t >> 4, columns (t & 15) * 4 .. +3 of the sub-block.
-// The sub-block is at (o, o) of D (row stride LD), pivots o .. o + nv - 1.  Row k
-// and column k do not change during step k (the diagonal is >= 0), so every
-// thread can update its strip in place; one barrier per pivot.
-template <int LD>
-__device__ __forceinline__ void lds_fw64(int32_t *D, int o, int nv) {
-  const int t = threadIdx.x;
-  const int i = o + (t >> 4), j = o + ((t & 15) << 2);
-  int4 *cp = reinterpret_cast<int4 *>(D + i * LD + j);
-  for (int k = o; k < o + nv; k++) {
-    const int a = D[i * LD + k];
-    const int4 b = *reinterpret_cast<const int4 *>(D + k * LD + j);
-    int4 c = *cp;
-    c.x = imin(c.x, a + b.x);
-    c.y = imin(c.y, a + b.y);
-    c.z = imin(c.z, a + b.z);
-    c.w = imin(c.w, a + b.w);
-    *cp = c;
-    __syncthreads();
-  }
-}
+// 64 x 64 blocks held in registers: a workgroup of 1024 / NC threads (NC = 4
+// or 2), thread t the 4 x NC cells at rows 4 (t / (64 / NC)), columns
+// NC (t % (64 / NC)); rows and columns past the matrix hold INF.  A SIMD
+// issues one wave's VALU instructions at half its rate, so a workgroup alone
+// on its CU wants two waves per SIMD (NC = 2: 512 threads); NC = 4 is for
+// closures that run beside other workgroups.
+template <int NC>
+struct Blk64 {
+  static constexpr int TPR = 64 / NC;  // threads per four rows
+  __device__ static __forceinline__ int ty() { return (int)threadIdx.x / TPR; }
+  __device__ static __forceinline__ int tx() { return (int)threadIdx.x % TPR; }
 
-
-constexpr int BLK_LD = 64 + 4;
-constexpr int BLK_LDS_WORDS = 64 * BLK_LD;
-
-__device__ __forceinline__ void close_block64(int32_t *blk, int64_t ld, int kb, int32_t *D) {
-  const int t = threadIdx.x;
-  for (int idx = t; idx < 64 * 64; idx += MP_THREADS) {
-    const int i = idx >> 6, j = idx & 63;
-    D[i * BLK_LD + j] = (i < kb && j < kb) ? blk[(int64_t)i * ld + j] : kInf;
-  }
-  __syncthreads();
-  const int r0 = t >> 4, j = (t & 15) << 2;
-  for (int k = 0; k < kb; k++) {
-    const int4 b = *reinterpret_cast<const int4 *>(D + k * BLK_LD + j);
+  template <int E>
+  __device__ static __forceinline__ void get(const int32_t *p, int (&v)[E]) {
+    typedef int vec __attribute__((ext_vector_type(E)));
+    const vec x = *reinterpret_cast<const vec *>(p);
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int i = r0 + 16 * q;
-      const int a = D[i * BLK_LD + k];
-      int4 *cp = reinterpret_cast<int4 *>(D + i * BLK_LD + j);
-      int4 c = *cp;
-      c.x = imin(c.x, a + b.x);
-      c.y = imin(c.y, a + b.y);
-      c.z = imin(c.z, a + b.z);
-      c.w = imin(c.w, a + b.w);
-      *cp = c;
-    }
-    __syncthreads();
+    for (int i = 0; i < E; i++) v[i] = x[i];
   }
-  for (int idx = t; idx < 64 * 64; idx += MP_THREADS) {
-    const int i = idx >> 6, j2 = idx & 63;
-    if (i < kb && j2 < kb) blk[(int64_t)i * ld + j2] = D[i * BLK_LD + j2];
+  template <int E>
+  __device__ static __forceinline__ void put(int32_t *p, const int (&v)[E]) {
+    typedef int vec __attribute__((ext_vector_type(E)));
+    vec x;
+#pragma unroll
+    for (int i = 0; i < E; i++) x[i] = v[i];
+    *reinterpret_cast<vec *>(p) = x;
+  }
+
+  // This thread's cells of a block with `rows` x `cols` valid cells (>= 1
+  // each), the others INF: vector loads (at any alignment) of a full block,
+  // else clamped addresses, so that neither form branches per cell.
+  __device__ static __forceinline__ void load(const int32_t *blk, int64_t ld, int rows, int cols,
+                                              int (&c)[4][NC]) {
+    typedef int vec __attribute__((ext_vector_type(NC), aligned(4)));
+    const int r = ty() * 4, j = tx() * NC;
+    if (rows == 64 && cols == 64) {
+      const int32_t *p = blk + (int64_t)r * ld + j;
+#pragma unroll
+      for (int i = 0; i < 4; i++, p += ld) {
+        const vec v = *reinterpret_cast<const vec *>(p);
+#pragma unroll
+        for (int q = 0; q < NC; q++) c[i][q] = v[q];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int32_t *p = blk + (int64_t)imin(r + i, rows - 1) * ld;
+#pragma unroll
+        for (int q = 0; q < NC; q++) {
+          const int v = p[imin(j + q, cols - 1)];
+          c[i][q] = (r + i < rows && j + q < cols) ? v : kInf;
+        }
+      }
+    }
+  }
+
+  __device__ static __forceinline__ void store(int32_t *blk, int64_t ld, int rows, int cols,
+                                               const int (&c)[4][NC]) {
+    typedef int vec __attribute__((ext_vector_type(NC), aligned(4)));
+    const int r = ty() * 4, j = tx() * NC;
+    int32_t *p = blk + (int64_t)r * ld + j;
+    if (rows == 64 && cols == 64) {
+#pragma unroll
+      for (int i = 0; i < 4; i++, p += ld) {
+        vec v;
+#pragma unroll
+        for (int q = 0; q < NC; q++) v[q] = c[i][q];
+        *reinterpret_cast<vec *>(p) = v;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; i++, p += ld)
+#pragma unroll
+        for (int q = 0; q < NC; q++)
+          if (r + i < rows && j + q < cols) p[q] = c[i][q];
+    }
+  }
+
+  // The block in LDS (row stride T64_LD) for products from there.
+  __device__ static __forceinline__ void to_lds(int32_t *T, const int (&c)[4][NC]);
+  // acc = min(acc, A (x) B) of two such blocks, whole in LDS: a product of a
+  // chain waits for memory once, not once per chunk of k.
+  __device__ static __forceinline__ void product(const int32_t *A, const int32_t *B,
+                                                 int (&acc)[4][NC]);
+
+  // ---- closure ----
+  // Two pivots p, q per step, one barrier: with the rows R0, R1 and columns
+  // C0, C1 of both as they stand before the step, row q after pivot p is
+  // min(R1, D[q][p] + R0), its column likewise, and a cell takes both pivots
+  // in one v_min3.  (A pivot does not change its own row and column: the
+  // diagonal is >= 0.)  Only the next two rows and columns go through LDS;
+  // with the whole block there each pivot moved it twice through 128 bytes
+  // per clock.  The chain of 32 steps is latency: 760 cycles each with 512
+  // threads, of which LDS write, barrier and read take 480 without any
+  // arithmetic (24,400 cycles a closure; the diagonal kernel at n = 1024 16.7
+  // -> 12.2 us, a 64-deep product from LDS 8,000 cycles).  The closure does not depend on the
+  // order of the pivots, so they go by their place in a thread's four rows:
+  // a step updates the next place's row and column first, publishes the next
+  // pivots, and does its other cells while the next reads are in flight.
+  struct Pivots {
+    int R0[NC], R1[NC], C0[4], C1[4], d01, d10;
+    // q: thread row of the second pivot; P its place; h = column place / NC
+    __device__ __forceinline__ void read(const int32_t *rd, int q, int P, int h) {
+      get<NC>(rd + NC * tx(), R0);
+      get<4>(rd + 128 + 4 * ty(), C0);
+      d01 = rd[4 * q + NC * h + (NC == 4 ? P : (P & 1))];
+      d10 = rd[128 + 4 * q + P];
+      get<NC>(rd + 64 + NC * tx(), R1);
+      get<4>(rd + 192 + 4 * ty(), C1);
+    }
+    __device__ __forceinline__ void derive() {
+#pragma unroll
+      for (int i = 0; i < NC; i++) R1[i] = imin(R1[i], d10 + R0[i]);
+#pragma unroll
+      for (int i = 0; i < 4; i++) C1[i] = imin(C1[i], C0[i] + d01);
+    }
+    // The cells of row or column P (FIRST), or all others.  The asm is
+    // volatile to keep the two groups on their sides of the barrier.
+    template <int P, bool FIRST>
+    __device__ __forceinline__ void update(int (&c)[4][NC]) const {
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < NC; j++)
+          if ((i == P || j == P) == FIRST) {
+            int t0, t1;
+            asm volatile(
+                "v_add_u32 %1, %3, %4\n\tv_add_u32 %2, %5, %6\n\tv_min3_i32 %0, %0, %1, %2"
+                : "+v"(c[i][j]), "=&v"(t0), "=&v"(t1)
+                : "v"(C0[i]), "v"(R0[j]), "v"(C1[i]), "v"(R1[j]));
+          }
+    }
+  };
+
+  // Row and column P of the cells of thread rows g, g + 1; h as above.
+  template <int P>
+  __device__ static __forceinline__ void publish(const int (&c)[4][NC], int32_t *wr, int g, int h) {
+    const int dy = ty() - g;
+    if (dy == 0 || dy == 1) put<NC>(wr + 64 * dy + NC * tx(), c[P]);
+    const int x0 = tx() - (4 / NC) * g - h;
+    if (x0 == 0 || x0 == 4 / NC) {
+      const int col[4] = {c[0][P], c[1][P], c[2][P], c[3][P]};
+      put<4>(wr + 128 + (x0 ? 64 : 0) + 4 * ty(), col);
+    }
+  }
+
+  // One step: `s` holds its pivots; leaves the next step's (place P, thread
+  // row g) in `s`, read from `next`.
+  template <int P>
+  __device__ static __forceinline__ void step(int (&c)[4][NC], Pivots &s, int32_t *next, int g,
+                                              int h) {
+    const Pivots cur = s;
+    cur.template update<P, true>(c);
+    publish<P>(c, next, g, h);
+    __syncthreads();
+    s.read(next, g + 1, P, h);
+    cur.template update<P, false>(c);
+    s.derive();
+  }
+
+  template <int E>
+  __device__ static __forceinline__ void rotate(int (&v)[E]) {
+    const int x = v[0];
+#pragma unroll
+    for (int i = 0; i + 1 < E; i++) v[i] = v[i + 1];
+    v[E - 1] = x;
+  }
+
+  // Closure by pivots 0 .. nv - 1 (nv >= 1); `buf` holds CLOSE64_WORDS ints.
+  // The four places run the same code: the cells' rows and columns rotate by
+  // one after each, so that the current place is 0 and the next one 1.
+  __device__ static __forceinline__ void close(int (&c)[4][NC], int nv, int32_t *buf) {
+    const int G = (((nv + 3) >> 2) + 3) & ~3;  // thread rows with pivots, in fours
+    Pivots s;
+    publish<0>(c, buf, 0, 0);
+    __syncthreads();
+    s.read(buf, 1, 0, 0);
+    s.derive();
+#pragma unroll 1
+    for (int place = 0; place < 4; place++) {
+      const int h = NC == 4 ? 0 : place >> 1;
+#pragma unroll 1
+      for (int g = 0; g < G - 4; g += 4) {
+        step<0>(c, s, buf + 256, g + 2, h);
+        step<0>(c, s, buf, g + 4, h);
+      }
+      step<0>(c, s, buf + 256, G - 2, h);
+      step<1>(c, s, buf, 0, NC == 4 ? 0 : (place + 1) >> 1);  // (after the last place: not used)
+#pragma unroll
+      for (int i = 0; i < 4; i++) rotate<NC>(c[i]);
+#pragma unroll
+      for (int j = 0; j < NC; j++) {
+        const int x = c[0][j];
+        c[0][j] = c[1][j]; c[1][j] = c[2][j]; c[2][j] = c[3][j]; c[3][j] = x;
+      }
+      rotate<NC>(s.R0);
+      rotate<NC>(s.R1);
+      rotate<4>(s.C0);
+      rotate<4>(s.C1);
+    }
+    __syncthreads();  // the buffer is free again
+  }
+};
+
+constexpr int CLOSE64_WORDS = 2 * 4 * 64;
+constexpr int T64_LD = 64 + 4;
+constexpr int T64_WORDS = 64 * T64_LD;
+
+template <int NC>
+__device__ __forceinline__ void Blk64<NC>::to_lds(int32_t *T, const int (&c)[4][NC]) {
+  int32_t *p = T + ty() * 4 * T64_LD + tx() * NC;
+#pragma unroll
+  for (int i = 0; i < 4; i++) put<NC>(p + i * T64_LD, c[i]);
+}
+
+template <int NC>
+__device__ __forceinline__ void Blk64<NC>::product(const int32_t *A, const int32_t *B,
+                                                   int (&acc)[4][NC]) {
+  const int32_t *pa = A + ty() * 4 * T64_LD, *pb = B + tx() * NC;
+#pragma unroll 2
+  for (int k = 0; k < 64; k += 2) {
+    int a[4][2], b0[NC], b1[NC];
+#pragma unroll
+    for (int i = 0; i < 4; i++) get<2>(pa + i * T64_LD + k, a[i]);
+    get<NC>(pb + k * T64_LD, b0);
+    get<NC>(pb + (k + 1) * T64_LD, b1);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int j = 0; j < NC; j++) {
+        int t0, t1;
+        asm volatile("v_add_u32 %1, %3, %4\n\tv_add_u32 %2, %5, %6\n\tv_min3_i32 %0, %0, %1, %2"
+                     : "+v"(acc[i][j]), "=&v"(t0), "=&v"(t1)
+                     : "v"(a[i][0]), "v"(b0[j]), "v"(a[i][1]), "v"(b1[j]));
+      }
   }
 }
+
+// Closure of one diagonal block of up to 64 x 64 (kb valid rows and columns)
+// in global memory by 1024 / NC threads; `buf` holds CLOSE64_WORDS ints.
+template <int NC>
+__device__ __forceinline__ void close_block64(int32_t *blk, int64_t ld, int kb, int32_t *buf) {
+  int c[4][NC];
+  Blk64<NC>::load(blk, ld, kb, kb, c);
+  Blk64<NC>::close(c, kb, buf);
+  Blk64<NC>::store(blk, ld, kb, kb, c);
+}
+
 constexpr int MP_BM = MpBig::BM;
 constexpr int MP_BN = MpBig::BN;
 

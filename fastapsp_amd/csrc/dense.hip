@@ -5,7 +5,7 @@
 // MysubMatBuild_path (fap/utils/util_Myalgorithm.h:30-73) from all arcs --
 // INF, then every arc in CSR order (the last duplicate wins, :50), then a
 // zero diagonal (:67-72).  These kernels build that matrix for one graph or
-// for a batch of graphs in one pair of launches.
+// for a batch of graphs in one launch.
 #include <algorithm>
 #include <vector>
 
@@ -14,38 +14,63 @@
 
 namespace fapk {
 
-__device__ __forceinline__ int find_job(const DenseJob *jobs, int count, int64_t x, bool rows) {
-  int lo = 0, hi = count - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    const int64_t b = rows ? (int64_t)jobs[mid].row_base : jobs[mid].cell_base;
-    if (b <= x) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
+// A wave builds a row, 1,024 columns at a time in its own LDS buffer: INF,
+// the row's arcs one after another (the last duplicate wins; a wave's LDS
+// writes land in order), the diagonal, then out with 16-byte stores.  Bound:
+// writing the matrices once.  512 graphs (1.19 GB): 0.31 ms; 1.62 ms as a
+// fill kernel that searched its job and divided once per cell, followed by a
+// kernel with a thread per row of arcs.
+constexpr int DR_COLS = 1024, DR_WAVES = 4;
 
-__global__ void dense_fill_kernel(const DenseJob *__restrict__ jobs, int count, int64_t cells) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; x < cells; x += stride) {
-    const DenseJob &jb = jobs[find_job(jobs, count, x, false)];
-    const int64_t local = x - jb.cell_base;
-    const int i = (int)(local / jb.n), j = (int)(local - (local / jb.n) * jb.n);
-    jb.mat[(int64_t)i * jb.ld + j] = (i == j) ? 0 : 0x3FFFFFFF;
+__global__ __launch_bounds__(64 * DR_WAVES) void dense_rows_kernel(const DenseJob *__restrict__ jobs,
+                                                                   int count, int32_t rows) {
+  typedef int vec4 __attribute__((ext_vector_type(4), aligned(4)));
+  __shared__ __attribute__((aligned(16))) int32_t buf[DR_WAVES * DR_COLS];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  int32_t *w = buf + wave * DR_COLS;
+  for (int x = blockIdx.x * DR_WAVES + wave; x < rows; x += gridDim.x * DR_WAVES) {
+    int lo = 0, hi = count - 1;  // the job whose rows hold x
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (jobs[mid].row_base <= x) lo = mid;
+      else hi = mid - 1;
+    }
+    const DenseJob &jb = jobs[lo];
+    const int u = x - jb.row_base, n = jb.n;
+    int32_t *row = jb.mat + (int64_t)u * jb.ld;
+    const int e0 = jb.row_offset[u], e1 = jb.row_offset[u + 1];
+    const int2 *__restrict__ edges = jb.edges;
+    for (int c0 = 0; c0 < n; c0 += DR_COLS) {
+#pragma unroll
+      for (int i = 0; i < DR_COLS; i += 256)
+        *reinterpret_cast<int4 *>(w + i + 4 * lane) =
+            make_int4(0x3FFFFFFF, 0x3FFFFFFF, 0x3FFFFFFF, 0x3FFFFFFF);
+      for (int e = e0; e < e1; e += 64) {
+        const int2 ed = e + lane < e1 ? edges[e + lane] : make_int2(-1, 0);
+        const unsigned at = (unsigned)(ed.x - c0);
+        const int m = e1 - e < 64 ? e1 - e : 64;
+        for (int k = 0; k < m; k++)
+          if (lane == k && at < (unsigned)DR_COLS) w[at] = ed.y;
+      }
+      if (lane == 0 && (unsigned)(u - c0) < (unsigned)DR_COLS) w[u - c0] = 0;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const int m = n - c0 < DR_COLS ? n - c0 : DR_COLS;
+#pragma unroll
+      for (int i = 0; i < DR_COLS; i += 256) {
+        const int j = i + 4 * lane;
+        const vec4 v = *reinterpret_cast<const vec4 *>(w + j);
+        if (j + 4 <= m) {
+          *reinterpret_cast<vec4 *>(row + c0 + j) = v;
+        } else {
+#pragma unroll
+          for (int q = 0; q < 3; q++)
+            if (j + q < m) row[c0 + j + q] = v[q];
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
   }
-}
-
-__global__ void dense_arcs_kernel(const DenseJob *__restrict__ jobs, int count, int32_t rows) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= rows) return;
-  const DenseJob &jb = jobs[find_job(jobs, count, x, true)];
-  const int u = x - jb.row_base;
-  int32_t *row = jb.mat + (int64_t)u * jb.ld;
-  for (int e = jb.row_offset[u]; e < jb.row_offset[u + 1]; e++) {
-    const int2 ed = jb.edges[e];
-    row[ed.x] = ed.y;
-  }
-  row[u] = 0;
 }
 
 }  // namespace fapk
@@ -56,11 +81,9 @@ int launch_dense_jobs(fap_ctx *ctx, const fapk::DenseJob *d_jobs, int32_t njobs,
                       int64_t rows, hipStream_t s) {
   if (njobs <= 0 || cells <= 0) return FAP_OK;
   if (rows > INT32_MAX) return fail(FAP_E_ARG, "dense build: too many rows");
-  const int64_t blocks = std::min<int64_t>((cells + 255) / 256, (int64_t)ctx->num_cus * 32);
-  hipLaunchKernelGGL(fapk::dense_fill_kernel, dim3((unsigned)blocks), dim3(256), 0, s, d_jobs,
-                     njobs, cells);
-  FAP_CHECK_LAUNCH();
-  hipLaunchKernelGGL(fapk::dense_arcs_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0,
+  const int64_t blocks = std::min<int64_t>((rows + fapk::DR_WAVES - 1) / fapk::DR_WAVES,
+                                           (int64_t)ctx->num_cus * 32);
+  hipLaunchKernelGGL(fapk::dense_rows_kernel, dim3((unsigned)blocks), dim3(64 * fapk::DR_WAVES), 0,
                      s, d_jobs, njobs, (int32_t)rows);
   FAP_CHECK_LAUNCH();
   return FAP_OK;

@@ -40,7 +40,7 @@
 
 #include "batch_desc.h"
 #include "common.h"
-#include "minplus_tile.h"
+#include "mfma_tile.h"
 
 namespace fapk {
 
@@ -134,6 +134,29 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(8)))
   }
 }
 
+// Pair passes in 128 x 128 tiles, additions on the matrix cores
+// (mfma_tile.h): both pivots of the pair in one 128-deep product, a workgroup
+// per tile (a grid-stride loop over tiles spilled inside the k loop: 478 us a
+// launch).  512 uneven graphs: 452 us a launch in 64 x 64 integer tiles, 317
+// now; the batch with its dense build 18.3 -> 13.1 ms.
+__global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void fw_pair128_kernel(
+    const BatchJob *__restrict__ jobs, const BatchSeg *__restrict__ segs, int nseg) {
+  __shared__ __attribute__((aligned(16))) int32_t lds[MxBig::LDS_WORDS];
+  const int ti = blockIdx.x;
+  const BatchSeg sg = segs[find_seg(segs, nseg, ti)];
+  const BatchJob job = jobs[sg.job];
+  const int r = sg.kind_r >> 3, n = job.n;
+  const int64_t ld = job.ld;
+  int I, J;
+  pair128_tile(r, job.nb, ti - sg.first, &I, &J);
+  const int base = r * BT;
+  const int flags =
+      ((((uintptr_t)job.mat) & 15) == 0 && (ld & 3) == 0) ? (MP_VEC_A | MP_VEC_B | MP_VEC_C) : 0;
+  MxBig::run(job.mat + (int64_t)I * 128 * ld + base, ld, job.mat + (int64_t)base * ld + J * 128,
+             ld, job.mat + (int64_t)I * 128 * ld + J * 128, ld, imin(128, n - I * 128),
+             imin(128, n - J * 128), imin(128, n - base), true, flags, lds);
+}
+
 // XCD (accelerator complex die) the calling wave runs on: the XCC_ID
 // hardware register.  Each XCD has its own L2.
 __device__ __forceinline__ int xcc_id() { return __builtin_amdgcn_s_getreg((3 << 11) | 20) & 15; }
@@ -225,7 +248,8 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(6)))
     const int kind = tr.y & 7, r = tr.y >> 3;
     if (kind == TASK_DIAG) {
       const int base = r * BT;
-      close_block64<4>(job.mat + (int64_t)base * job.ld + base, job.ld, imin(BT, job.n - base), lds);
+      close_block64_call<4>((mp_out_ptr)(job.mat + (int64_t)base * job.ld + base), job.ld,
+                            imin(BT, job.n - base), (mp_lds_ptr)lds);
     } else {
       batch_tile_task(job, kind, r, tr.z, lds);
     }
@@ -261,6 +285,8 @@ __global__ void fw_queue_reset_kernel(int32_t *ctrl, int nctrl, int32_t *done, i
 }  // namespace fapk
 
 namespace fapi {
+
+constexpr int64_t kPair128MinTiles = 2 * 256;  // two per CU of an MI355X
 
 // Launch p of a batch holds phase p of every job that has one, jobs in
 // decreasing size (longest processing time first), each job's phase one
@@ -319,6 +345,30 @@ void build_fw_batch(int32_t count, int32_t *const *mats, const int32_t *n, const
     }
     out->launch_tasks.push_back(first);
     out->seg_off.push_back((int32_t)out->segs.size());
+  }
+  out->pair128_off.assign(launches, -1);
+  out->pair128_tasks.assign(launches, 0);
+  for (int L = 0; L < launches; L++) {
+    int64_t big = 0;
+    bool pair = out->launch_tasks[L] > 0;
+    for (int q = out->seg_off[L]; q < out->seg_off[L + 1]; q++) {
+      pair = pair && (out->segs[q].kind_r & 7) == fapk::TASK_REST2;
+      big += fapk::pair128_count(out->jobs[out->segs[q].job].nb);
+    }
+    // a 128 x 128 tile costs about 2.5 of the 64 x 64 ones: not worth it for
+    // jobs of 3 and 5 blocks, whose last 128-block is half empty, nor below
+    // two tiles per CU, where the shorter tiles end sooner (8 matrices of 512,
+    // 72 tiles: a 64 x 64 grid's parts 950 us in 64-tiles, 1,015 in 128)
+    if (!pair || 2 * (int64_t)out->launch_tasks[L] < 5 * big || big < kPair128MinTiles) continue;
+    out->pair128_off[L] = (int32_t)out->segs.size();
+    int32_t at = 0;
+    for (int q = out->seg_off[L]; q < out->seg_off[L + 1]; q++) {
+      const fapk::BatchSeg sg = out->segs[q];
+      const int cnt = fapk::pair128_count(out->jobs[sg.job].nb);
+      out->segs.push_back(fapk::BatchSeg{sg.job, sg.kind_r, at, cnt});
+      at += cnt;
+    }
+    out->pair128_tasks[L] = at;
   }
   out->key = fap_tune_key_batch(count, n);
 }
@@ -563,6 +613,9 @@ int launch_fw_batch(fap_ctx *ctx, const FwBatchDesc &desc, const fapk::BatchJob 
     else if (kind == fapk::TASK_REST)
       hipLaunchKernelGGL(fapk::fw_phase_kernel<fapk::TASK_REST>, grid, block, 0, s, d_jobs, sg,
                          nseg, cnt);
+    else if (kind == fapk::TASK_REST2 && desc.pair128_off[p] >= 0)
+      hipLaunchKernelGGL(fapk::fw_pair128_kernel, dim3(desc.pair128_tasks[p]), block, 0, s, d_jobs,
+                         d_segs + desc.pair128_off[p], nseg);
     else if (kind == fapk::TASK_REST2)
       hipLaunchKernelGGL(fapk::fw_phase_kernel<fapk::TASK_REST2>, grid, block, 0, s, d_jobs, sg,
                          nseg, cnt);
@@ -864,7 +917,11 @@ int fap_fw_batched_noalloc(fap_ctx *ctx, int32_t count, int32_t *const *d_mats, 
   build_fw_batch(count, d_mats, n, ld, &d);
   const size_t jobs_b = sizeof(fapk::BatchJob) * d.jobs.size();
   const size_t segs_off = (jobs_b + 255) & ~(size_t)255;
-  const size_t segs_b = sizeof(fapk::BatchSeg) * d.segs.size();
+  size_t segs_b = sizeof(fapk::BatchSeg) * d.segs.size();
+  if (segs_off + segs_b > (size_t)FAP_NOALLOC_SCRATCH_BYTES) {
+    d.drop_pair128();
+    segs_b = sizeof(fapk::BatchSeg) * d.segs.size();
+  }
   if (segs_off + segs_b > (size_t)FAP_NOALLOC_SCRATCH_BYTES)
     return fail(FAP_E_ARG, "fw_batched_noalloc: the batch's descriptors need " +
                                std::to_string(segs_off + segs_b) + " bytes, above the " +

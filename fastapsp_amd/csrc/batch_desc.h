@@ -122,6 +122,20 @@ __host__ __device__ inline void pair_tile(int r, int nb, int idx, int *I, int *J
   *J = j < r ? j : j + 2;
 }
 
+// The pair pass again in 128 x 128 tiles: pairs start at even blocks, so the
+// pivot pair is one block of 128 and the tiles off it are those of the other
+// 128-blocks (the last one may be half empty).
+__host__ __device__ inline int pair128_count(int nb) {
+  const int m = (nb + 1) / 2 - 1;
+  return m * m;
+}
+
+__host__ __device__ inline void pair128_tile(int r, int nb, int idx, int *I, int *J) {
+  const int m = (nb + 1) / 2 - 1, i = idx / m, j = idx - (idx / m) * m;
+  *I = i < r / 2 ? i : i + 1;
+  *J = j < r / 2 ? j : j + 1;
+}
+
 // Kernel instance that runs a task kind (the cross kinds run on the
 // single-pivot instance); every task of a launch runs on one instance.
 __host__ __device__ constexpr int kind_instance(int kind) {
@@ -150,6 +164,16 @@ struct FwBatchDesc {
   std::vector<fapk::BatchSeg> segs;
   std::vector<int32_t> seg_off;
   std::vector<int32_t> launch_tasks;
+  // pair passes in 128 x 128 tiles: launch p's segments start at pair128_off[p]
+  // (after every launch's own, as many as those), -1 where it has none
+  std::vector<int32_t> pair128_off;
+  std::vector<int32_t> pair128_tasks;
+  // Without them (pair passes then run in 64 x 64 tiles), where descriptor
+  // space is short.
+  void drop_pair128() {
+    segs.resize(seg_off.back());
+    pair128_off.assign(pair128_off.size(), -1);
+  }
   int64_t ops = 0;
   int64_t key = 0;  // tune cache bucket (fap_tune_key_batch)
 };

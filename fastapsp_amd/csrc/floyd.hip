@@ -77,13 +77,10 @@ __device__ __forceinline__ void close_block128(int32_t *blk, int64_t ld, int kb,
   B::store(p11, ld, n1, n1, d11);
 }
 
-// The closures as functions of their own, for kernels that reach them in one
-// workgroup: inlined, their cells would take registers from the tile loop.
-template <int T>
-__device__ __attribute__((noinline)) void close_block_call(mx_out_ptr blk, int64_t ld, int kb,
-                                                           mx_lds_ptr lds) {
-  if (T == 128) close_block128<4>((int32_t *)blk, ld, kb, (int32_t *)lds);
-  else close_block64<4>((int32_t *)blk, ld, kb, (int32_t *)lds);
+// As a function of its own, for the phase-3 kernel (as close_block64_call).
+__device__ __attribute__((noinline)) void close_block128_call(mp_out_ptr blk, int64_t ld, int kb,
+                                                              mp_lds_ptr lds) {
+  close_block128<4>((int32_t *)blk, ld, kb, (int32_t *)lds);
 }
 
 constexpr int FW_DIAG_THREADS = 512;  // workgroups alone on their CU: Blk64<2>
@@ -269,7 +266,8 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
   Tile::run(a, ld, b, ld, c, ld, imin(T, n - I * T), imin(T, n - J * T), kb, true, flags, lds);
   if (fuse && blockIdx.x == 0) {
     __syncthreads();  // the tile's writes above come before the closure reads it
-    close_block_call<T>((mx_out_ptr)c, ld, imin(T, n - I * T), (mx_lds_ptr)lds);
+    if (T == 64) close_block64_call<4>((mp_out_ptr)c, ld, imin(T, n - I * T), (mp_lds_ptr)lds);
+    else close_block128_call((mp_out_ptr)c, ld, imin(T, n - I * T), (mp_lds_ptr)lds);
   }
 }
 

@@ -50,19 +50,16 @@ __device__ __forceinline__ uint32_t mx_digits(uint32_t w) {
   return __umul24((w >> 11) & 0x7FFu, 65536u - 2048u) + w;
 }
 
-typedef __attribute__((address_space(3))) int32_t *mx_lds_ptr;
-typedef __attribute__((address_space(1))) const int32_t *mx_in_ptr;
-typedef __attribute__((address_space(1))) int32_t *mx_out_ptr;
 
 // The same tile with integer additions, as a function of its own: inlined,
 // its registers and the matrix tile's accumulators would be live together
 // (both spilled: 8192^3 on values that the digits do not hold took 42.8 ms;
 // 19.3 ms this way, 18.8 ms on the integer tile alone).
 template <int NI, int NJ>
-__device__ __attribute__((noinline)) void int_tile(mx_in_ptr A, int64_t lda, mx_in_ptr B,
-                                                   int64_t ldb, mx_out_ptr C, int64_t ldc,
+__device__ __attribute__((noinline)) void int_tile(mp_in_ptr A, int64_t lda, mp_in_ptr B,
+                                                   int64_t ldb, mp_out_ptr C, int64_t ldc,
                                                    int m_valid, int n_valid, int K,
-                                                   bool accumulate, int flags, mx_lds_ptr lds) {
+                                                   bool accumulate, int flags, mp_lds_ptr lds) {
   __syncthreads();
   MpTile<4 * NI, 4 * NJ>::run((const int32_t *)A, lda, (const int32_t *)B, ldb, (int32_t *)C, ldc,
                               m_valid, n_valid, K, accumulate, flags, (int32_t *)lds);
@@ -251,8 +248,8 @@ struct MxTile {
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[i][j][r] = 0x7F800000;  // above every sum: INF
     if (!fits(lda, ldb, n_valid, K) || product(A, lda, B, ldb, m_valid, n_valid, K, lds, acc)) {
-      int_tile<NI, NJ>((mx_in_ptr)A, lda, (mx_in_ptr)B, ldb, (mx_out_ptr)C, ldc, m_valid, n_valid,
-                       K, accumulate, flags, (mx_lds_ptr)lds);
+      int_tile<NI, NJ>((mp_in_ptr)A, lda, (mp_in_ptr)B, ldb, (mp_out_ptr)C, ldc, m_valid, n_valid,
+                       K, accumulate, flags, (mp_lds_ptr)lds);
       return;
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;

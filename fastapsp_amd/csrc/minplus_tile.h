@@ -33,6 +33,11 @@ constexpr int MP_BK = 16;
 constexpr int MP_THREADS = 256;
 constexpr int MP_AS_LD = MP_BK + 4;  // words per A row in LDS
 
+// Pointers of functions that are not inlined keep their address spaces.
+typedef __attribute__((address_space(3))) int32_t *mp_lds_ptr;
+typedef __attribute__((address_space(1))) const int32_t *mp_in_ptr;
+typedef __attribute__((address_space(1))) int32_t *mp_out_ptr;
+
 // Flags describing what 16-byte vector accesses are legal for a launch.
 enum : int {
   MP_VEC_A = 1,  // A base 16-byte aligned and lda % 4 == 0
@@ -509,6 +514,14 @@ __device__ __forceinline__ void close_block64(int32_t *blk, int64_t ld, int kb, 
   Blk64<NC>::load(blk, ld, kb, kb, c);
   Blk64<NC>::close(c, kb, buf);
   Blk64<NC>::store(blk, ld, kb, kb, c);
+}
+
+// The same as a function of its own, for kernels that reach it beside a tile
+// loop: inlined, its cells would take registers from the loop.
+template <int NC>
+__device__ __attribute__((noinline)) void close_block64_call(mp_out_ptr blk, int64_t ld, int kb,
+                                                             mp_lds_ptr buf) {
+  close_block64<NC>((int32_t *)blk, ld, kb, (int32_t *)buf);
 }
 
 constexpr int MP_BM = MpBig::BM;

@@ -432,6 +432,8 @@ int launch_wave(fap_server *S, Lane &L) {
     build_fw_batch((int32_t)bmats.size(), bmats.data(), bns.data(), blds.data(), &fd);
     const size_t o_dj = put(dj.data(), sizeof(fapk::DenseJob) * dj.size());
     const size_t o_bj = put(fd.jobs.data(), sizeof(fapk::BatchJob) * fd.jobs.size());
+    if (off + sizeof(fapk::BatchSeg) * fd.segs.size() > (size_t)S->opts.stage_bytes)
+      fd.drop_pair128();
     const size_t o_sg = put(fd.segs.data(), sizeof(fapk::BatchSeg) * fd.segs.size());
     if (off > (size_t)S->opts.stage_bytes) return fail(FAP_E_NOMEM, "wave staging overflow");
     FAP_HIP(hipMemcpyAsync(L.d_stage, h, off, hipMemcpyHostToDevice, s));

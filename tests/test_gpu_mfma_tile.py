@@ -79,3 +79,56 @@ def test_closure_values(gpu_ctx, n, hi):
         gpu_ctx.set_option("fw_tile", 0)
     np.testing.assert_array_equal(d.get(), O.floyd(m))
     d.free()
+
+
+@pytest.mark.parametrize("sizes", [[449, 512] + [500] * 56, [385, 64, 130, 700] * 16, [321] * 128,
+                                   [256] * 511])
+@pytest.mark.parametrize("hi,pad", [(1000, 0), (1 << 25, 3)])
+def test_batched_pair_passes(gpu_ctx, sizes, hi, pad):
+    """Batches with enough tiles for pair passes in 128 x 128 tiles, and two that keep 64 x 64 (jobs
+    of 321: half-empty last blocks; 511 jobs of one 128-tile each: too few)."""
+    rng = np.random.default_rng(sum(sizes) + hi)
+    mats = []
+    for n in sizes:
+        m = values(rng, (n, n), hi, 0.95)
+        np.fill_diagonal(m, 0)
+        buf = np.full((n, n + pad), -3, np.int32)
+        buf[:, :n] = m
+        mats.append((m, gpu_ctx.to_device(buf)))
+    gpu_ctx.fw_batched([d.ptr for _, d in mats], sizes, [n + pad for n in sizes])
+    for i, (m, d) in enumerate(mats):
+        n = m.shape[0]
+        got = d.get()
+        if i % 8:  # the oracle closes every eighth
+            d.free()
+            continue
+        np.testing.assert_array_equal(got[:, :n], O.floyd(m))
+        assert (got[:, n:] == -3).all()
+        d.free()
+
+
+@pytest.mark.parametrize("n", [1, 3, 70, 1023, 1025, 2050])
+def test_dense_rows(gpu_ctx, n):
+    """Dense matrices from CSRs: row lengths around the 1,024-column pieces, more than 64 arcs in a
+    row, duplicates (the last wins), self loops, an unaligned stride."""
+    import fastapsp_amd as fa
+    rng = np.random.default_rng(n)
+    want = np.full((n, n + 1), -8, np.int32)
+    want[:, :n] = INF
+    ro, col, w = [0], [], []
+    for u in range(n):
+        k = int(rng.integers(0, 8)) if u % 17 else 150
+        c, x = rng.integers(0, n, k), rng.integers(0, 1000, k)
+        for a, b in zip(c, x):
+            want[u, a] = b
+        want[u, u] = 0
+        col += list(c)
+        w += list(x)
+        ro.append(len(col))
+    g = fa.DeviceGraph(gpu_ctx, np.array(ro, np.int32), np.array(col, np.int32),
+                       np.array(w, np.int32))
+    d = gpu_ctx.to_device(np.full((n, n + 1), -8, np.int32))
+    gpu_ctx.dense_from_graphs([g], [d.ptr], [n + 1])
+    np.testing.assert_array_equal(d.get(), want)
+    d.free()
+    g.close()

@@ -1,0 +1,77 @@
+"""The boundary index's matrix-core tiles at their edges: border lists longer than one LDS piece, lists
+shorter than a chunk, values past the digits.  Rows equal to the oracle's per-part pipeline."""
+
+import numpy as np
+import pytest
+
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+
+def solve_all(gpu_ctx, ro, col, w, gid, K):
+    """Row blocks of every part through one batched call, and the oracle's preconditioning."""
+    V = len(ro) - 1
+    pc = O.precondition(K, gid, ro, col)
+    dg = gpu_ctx.upload_graph(ro, col, w)
+    dg.set_partition(gid, pc["st2ed"], pc["ed2st"])
+    assert dg.build_index()
+    ids = list(range(1, K + 1))
+    outs = [gpu_ctx.alloc((int(pc["ver_num"][p]), V)) for p in ids]
+    dg.subgraph_solve_batch([int(pc["ver_off"][p]) for p in ids], [int(pc["ver_num"][p]) for p in ids],
+                            [int(pc["bdy_num"][p]) for p in ids], [o.ptr for o in outs], V)
+    got = [o.get() for o in outs]
+    for o in outs:
+        o.free()
+    dg.close()
+    return got, pc
+
+
+def random_digraph(V, degree, whi, seed):
+    rng = np.random.default_rng(seed)
+    u = np.repeat(np.arange(V), degree)
+    v = rng.integers(0, V, V * degree)
+    keep = u != v
+    key = np.unique(u[keep] * V + v[keep])
+    u, v = key // V, key % V
+    w = rng.integers(1, whi + 1, u.size).astype(np.int32)
+    ro = np.zeros(V + 1, np.int32)
+    np.cumsum(np.bincount(u, minlength=V), out=ro[1:])
+    return ro, v.astype(np.int32), w
+
+
+# 900 vertices a part, nearly all on its border: lists of ~900 positions (two pieces); 521 and 520
+# around the longest list that stays in one piece; 1 << 24: integer additions
+@pytest.mark.parametrize("V,K,whi", [(1800, 2, 100), (1800, 2, 1 << 24), (1042, 2, 50), (1040, 2, 50),
+                                     (1500, 3, 255)])
+def test_long_border_lists(gpu_ctx, V, K, whi):
+    ro, col, w = random_digraph(V, 6, whi, V + K)
+    gid = (np.arange(V) * K // V + 1).astype(np.int32)
+    got, pc = solve_all(gpu_ctx, ro, col, w, gid, K)
+    for p in range(1, K + 1):
+        np.testing.assert_array_equal(got[p - 1], O.run_part(p, ro, col, w, gid, pc))
+
+
+# a path of cliques: borders of one vertex, lists of one or two positions
+def test_short_border_lists(gpu_ctx):
+    K, n = 9, 30
+    V = K * n
+    arcs = []
+    rng = np.random.default_rng(4)
+    for p in range(K):
+        for i in range(n):
+            for j in rng.integers(0, n, 4):
+                if i != j:
+                    arcs.append((p * n + i, p * n + int(j)))
+        if p:
+            arcs += [(p * n, p * n - 1), (p * n - 1, p * n)]
+    arcs = sorted(set(arcs))
+    u = np.array([a for a, _ in arcs])
+    ro = np.zeros(V + 1, np.int32)
+    np.cumsum(np.bincount(u, minlength=V), out=ro[1:])
+    col = np.array([b for _, b in arcs], np.int32)
+    w = rng.integers(1, 1000, len(arcs)).astype(np.int32)
+    gid = (np.arange(V) // n + 1).astype(np.int32)
+    got, pc = solve_all(gpu_ctx, ro, col, w, gid, K)
+    for p in range(1, K + 1):
+        np.testing.assert_array_equal(got[p - 1], O.run_part(p, ro, col, w, gid, pc))

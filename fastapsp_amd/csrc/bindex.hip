@@ -27,7 +27,8 @@
 //     too small).  The iterations run on the device: a one-workgroup
 //     scheduling step lists each iteration's tiles, and the host only
 //     checks for convergence every few iterations.  On the 512x512 grid cut
-//     in 256 parts, 32 parts per call: ~224 iterations.
+//     in 256 parts, 32 parts per call: ~224 iterations -- a graph of that many
+//     parts takes step 1 from the index's coarse level instead (hindex.hip).
 //  2. expansion.  A path from s to v in part Q enters Q for the last time at
 //     a boundary vertex c of Q (or starts there: s is one), then stays in Q:
 //     d(s, v) = min over c in B_Q of d_H(s, c) + L_Q(c, v).  Per part that
@@ -108,6 +109,7 @@ struct fap_bidx {
   std::vector<BidxPart> h_parts;          // host copy, index = part id - 1
   std::vector<int32_t> h_hpos;            // H position of each boundary vertex (local index order)
   std::vector<int32_t> boff;              // K + 1: each part's first entry in h_hpos
+  std::vector<fapi::BidxCut> h_cuts;      // cut arcs between H ids
   BidxPart *parts = nullptr;       // device, K
   int32_t *in_off = nullptr;       // nbp + 1: cut arcs into each H id
   int2 *in_arc = nullptr;          // {source H id, weight}
@@ -701,6 +703,63 @@ constexpr int32_t kMaxIndexH = 1 << 18;  // boundary vertices (H ids): X rows of
 
 }  // namespace
 
+void bidx_free(fap_bidx *x) { free_bidx(x); }
+
+void bidx_describe(const fap_bidx *x, BidxDesc *out) {
+  out->K = x->K;
+  out->nbp = x->nbp;
+  out->nb = x->nb;
+  out->parts.clear();
+  for (const BidxPart &P : x->h_parts)
+    out->parts.push_back(BidxPartDesc{P.start, P.n, P.b, P.hoff, P.lbb_off, P.ldb});
+  out->cuts = &x->h_cuts;
+  out->hpos = &x->h_hpos;
+  out->boff = &x->boff;
+  out->lbb = x->lbb;
+  out->bytes = x->bytes;
+}
+
+int bidx_coarse(const std::vector<BidxPartDesc> &regions, const std::vector<int32_t> &colid,
+                int32_t *D, int32_t nbp, hipStream_t s, fap_bidx **out) {
+  *out = nullptr;
+  fap_bidx *x = new fap_bidx();
+  x->K = (int32_t)regions.size();
+  x->nbp = nbp;
+  std::vector<int2> ctiles;
+  for (int32_t q = 0; q < x->K; q++) {
+    const BidxPartDesc &r = regions[q];
+    x->h_parts.push_back(BidxPart{r.start, r.n, r.b, r.hoff, 0, r.lbb_off, 0, r.ldb});
+    x->nb += r.b;
+    for (int32_t j = 0; j < r.n; j += kExpandCols) ctiles.push_back(make_int2(q, j));
+  }
+  x->nctiles = (int32_t)ctiles.size();
+  int rc = upload(x->h_parts, &x->parts, &x->bytes, s);
+  if (rc == FAP_OK) rc = upload(colid, &x->colid, &x->bytes, s);
+  if (rc == FAP_OK) rc = upload(ctiles, &x->ctiles, &x->bytes, s);
+  const hipError_t e = hipStreamSynchronize(s);  // the uploads read host vectors of this call
+  if (rc == FAP_OK && e != hipSuccess) rc = hip_fail(e, "coarse index", __FILE__, __LINE__);
+  if (rc != FAP_OK) {
+    free_bidx(x);
+    return rc;
+  }
+  x->lbv = D;
+  *out = x;
+  return FAP_OK;
+}
+
+const int32_t *bidx_columns(const fap_bidx *x) { return x->colid; }
+
+// Rows of X to every column: rowptr[r][colid] from X's boundary distances.
+int bidx_expand(const fap_bidx *x, const int32_t *X, int64_t ldx, int32_t nsrc,
+                int32_t *const *d_rowptr, hipStream_t s) {
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(fapk::bidx_expand_kernel<kExpandTM, kExpandTN>),
+                     dim3(x->nctiles, (nsrc + 16 * kExpandTM - 1) / (16 * kExpandTM)),
+                     dim3(fapk::MP_THREADS), 0, s, X, ldx, nsrc, d_rowptr, x->ctiles, x->parts,
+                     x->lbv, x->colid);
+  FAP_CHECK_LAUNCH();
+  return FAP_OK;
+}
+
 void bidx_release(fap_graph_dev *g) {
   free_bidx(g->bidx);
   g->bidx = nullptr;
@@ -835,6 +894,7 @@ int bidx_build(fap_ctx *ctx, fap_graph_dev *g) {
         const int32_t v = ed[e].x;
         if (gid[v] == gid[u]) continue;
         lists[hid[v]].push_back(make_int2(hid[u], ed[e].y));
+        x->h_cuts.push_back(BidxCut{hid[u], hid[v], ed[e].y, gid[u] - 1, gid[v] - 1});
         cuts[gid[v] - 1].push_back({gid[u] - 1, hid[v] - x->h_parts[gid[v] - 1].hoff});
       }
     in1.assign(x->nbp, make_int2(-1, 0));
@@ -1060,12 +1120,7 @@ int bidx_rows(fap_ctx *ctx, const fap_graph_dev *g, int32_t count, const int32_t
     FAP_HIP(hipStreamSynchronize(s));
     if (hc[BC_DONE]) break;
   }
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(fapk::bidx_expand_kernel<kExpandTM, kExpandTN>),
-                     dim3(x->nctiles, (nsrc + 16 * kExpandTM - 1) / (16 * kExpandTM)),
-                     dim3(fapk::MP_THREADS), 0, s, X, ldx, nsrc, d_rowptr, x->ctiles, x->parts,
-                     x->lbv, x->colid);
-  FAP_CHECK_LAUNCH();
-  return FAP_OK;
+  return bidx_expand(x, X, ldx, nsrc, d_rowptr, s);
 }
 
 int32_t bidx_part(const fap_graph_dev *g, int32_t start, int32_t n, int32_t b) {
@@ -1078,20 +1133,3 @@ int32_t bidx_part(const fap_graph_dev *g, int32_t start, int32_t n, int32_t b) {
 }
 
 }  // namespace fapi
-
-using namespace fapi;
-
-extern "C" int fap_graph_build_index(fap_ctx *ctx, fap_graph_dev *g, int32_t *built) {
-  if (!ctx || !g) return fail(FAP_E_ARG, "null ctx/graph");
-  FAP_HIP(hipSetDevice(ctx->device));
-  FAP_TRY(bidx_build(ctx, g));
-  if (built) *built = g->bidx ? 1 : 0;
-  return FAP_OK;
-}
-
-extern "C" int fap_graph_index_info(const fap_graph_dev *g, int32_t *boundary, int64_t *bytes) {
-  if (!g) return fail(FAP_E_ARG, "null graph");
-  if (boundary) *boundary = g->bidx ? g->bidx->nb : 0;
-  if (bytes) *bytes = g->bidx ? (int64_t)g->bidx->bytes : 0;
-  return FAP_OK;
-}

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -50,6 +51,7 @@ struct Workspace {
 }  // namespace fapi
 
 struct fap_bidx;  // boundary index of a partitioned graph (bindex.hip)
+struct fap_hidx;  // its coarse level, regions of parts (hindex.hip)
 
 struct fap_graph_dev {
   int32_t V = 0;
@@ -68,6 +70,10 @@ struct fap_graph_dev {
   std::vector<int32_t> h_graph_id;  // host copy of graph_id (part range checks)
   fap_bidx *bidx = nullptr;         // built on first batched part solve (bindex.hip)
   int bidx_state = 0;               // 0 not tried, 1 built, -1 not applicable
+  std::atomic<fap_hidx *> hidx{nullptr};  // with bidx, where the graph has enough parts
+  std::mutex index_mu;              // held while either is built: contexts may share a graph
+  bool hidx_tried = false;
+  int64_t batch_parts = 0;          // parts solved through the index before its coarse level
 };
 
 struct fap_ctx {
@@ -88,6 +94,7 @@ struct fap_ctx {
   fapi::Workspace ws_srcs;    // batched-solve sources and row pointers
   fapi::Workspace ws_bidx;    // boundary distances of a batched solve's sources
   fapi::Workspace ws_bbf;     // boundary iterations: tile lists and changed flags
+  fapi::Workspace ws_hidx;    // region-boundary distances of a batched solve's sources
   uint32_t *host_pinned = nullptr;  // small pinned host buffer for counters
   void *host_bbf = nullptr;         // pinned staging of the boundary iterations
   size_t host_bbf_bytes = 0;
@@ -156,6 +163,40 @@ int bidx_build(fap_ctx *ctx, fap_graph_dev *g);
 int bidx_rows(fap_ctx *ctx, const fap_graph_dev *g, int32_t count, const int32_t *qidx,
               const int32_t *rowoff, int32_t nsrc, int32_t *const *d_rowptr, hipStream_t s);
 void bidx_release(fap_graph_dev *g);
+// Parts of the index as its coarse level (hindex.hip) uses them.
+struct BidxCut {  // arc u -> v of length w between H ids of parts pu != pv
+  int32_t u, v, w, pu, pv;
+};
+struct BidxPartDesc {  // a part (or region): n columns, the first H id of its b boundary vertices,
+  int32_t start, n, b, hoff;  // and where its local distances are (row stride ldb)
+  int64_t lbb_off;
+  int32_t ldb;
+};
+struct BidxDesc {
+  int32_t K = 0, nbp = 0, nb = 0;
+  std::vector<BidxPartDesc> parts;
+  const std::vector<BidxCut> *cuts = nullptr;
+  const std::vector<int32_t> *hpos = nullptr, *boff = nullptr;  // H positions of boundary vertices
+  const int32_t *lbb = nullptr;                                 // device
+  size_t bytes = 0;
+};
+void bidx_describe(const fap_bidx *x, BidxDesc *out);
+// An index over regions that serves expansions only: region r's b boundary
+// rows of D (device, owned by the result on success), columns `colid` (device:
+// bidx_columns).
+int bidx_coarse(const std::vector<BidxPartDesc> &regions, const std::vector<int32_t> &colid,
+                int32_t *D, int32_t nbp, hipStream_t s, fap_bidx **out);
+const int32_t *bidx_columns(const fap_bidx *x);
+int bidx_expand(const fap_bidx *x, const int32_t *X, int64_t ldx, int32_t nsrc,
+                int32_t *const *d_rowptr, hipStream_t s);
+void bidx_free(fap_bidx *x);
+// Coarse level (hindex.hip): built beside the index where it pays (leaves
+// g->hidx null otherwise), stage-1 rows through it or, without one, through
+// bidx_rows; release.
+int hidx_build(fap_ctx *ctx, fap_graph_dev *g, hipStream_t s);
+int hidx_rows(fap_ctx *ctx, const fap_graph_dev *g, int32_t count, const int32_t *qidx,
+              const int32_t *rowoff, int32_t nsrc, int32_t *const *d_rowptr, hipStream_t s);
+void hidx_release(fap_graph_dev *g);
 // Index of the part starting at st2ed offset `start` with n vertices and b
 // boundary ones, or -1 when the index does not hold that part as given.
 int32_t bidx_part(const fap_graph_dev *g, int32_t start, int32_t n, int32_t b);

@@ -202,7 +202,7 @@ int fap_ctx_destroy(fap_ctx *ctx) {
   (void)hipStreamSynchronize(ctx->stream);
   Workspace *all[] = {&ctx->ws_sub, &ctx->ws_queue, &ctx->ws_stamp, &ctx->ws_small,
                       &ctx->ws_misc, &ctx->ws_batch, &ctx->ws_dense, &ctx->ws_srcs,
-                      &ctx->ws_bidx, &ctx->ws_bbf};
+                      &ctx->ws_bidx, &ctx->ws_bbf, &ctx->ws_hidx};
   for (Workspace *w : all)
     if (w->ptr) (void)hipFree(w->ptr);
   if (ctx->host_pinned) (void)hipHostFree(ctx->host_pinned);
@@ -512,6 +512,7 @@ int fap_graph_set_partition(fap_ctx *ctx, fap_graph_dev *g, const int32_t *graph
   FAP_HIP(hipStreamSynchronize(ctx->stream));
   g->h_st2ed.assign(st2ed, st2ed + V);
   g->h_graph_id.assign(graph_id, graph_id + V);
+  hidx_release(g);
   bidx_release(g);  // an index belongs to the partition it was built for
   return FAP_OK;
 }
@@ -519,6 +520,7 @@ int fap_graph_set_partition(fap_ctx *ctx, fap_graph_dev *g, const int32_t *graph
 int fap_graph_free(fap_ctx *ctx, fap_graph_dev *g) {
   if (!g) return FAP_OK;
   if (ctx) (void)hipSetDevice(ctx->device);
+  hidx_release(g);
   bidx_release(g);
   int32_t *bufs[] = {g->row_offset, g->graph_id, g->st2ed, g->ed2st, g->in_offset};
   for (int32_t *b : bufs)

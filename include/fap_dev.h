@@ -311,8 +311,11 @@ int fap_subgraph_pred(fap_ctx *ctx, fap_graph_dev *g, int32_t start, int32_t n_s
  * first batched solve (option "sssp_index"); this call builds it at once.
  * *built = 0 when the graph does not qualify (more than ~36 k boundary
  * vertices, duplicate arcs, a partition whose parts do not list their
- * boundary vertices first); stage 1 then runs fap_sssp_multi.  The index is
- * dropped by fap_graph_set_partition and fap_graph_free.  Synchronous. */
+ * boundary vertices first); stage 1 then runs fap_sssp_multi.  A graph of 32
+ * parts or more also gets the index's coarse level (regions of parts, closed;
+ * stage 1 without iterations), here or with the batched solve that brings the
+ * parts solved to 32, unless it is too large or leaves most boundary vertices
+ * on a region's border.  The index is dropped by fap_graph_set_partition and fap_graph_free.  Synchronous. */
 int fap_graph_build_index(fap_ctx *ctx, fap_graph_dev *g, int32_t *built);
 /* boundary vertices held by the index (0 without one) and its device bytes */
 int fap_graph_index_info(const fap_graph_dev *g, int32_t *boundary, int64_t *bytes);

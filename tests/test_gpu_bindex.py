@@ -75,3 +75,53 @@ def test_short_border_lists(gpu_ctx):
     got, pc = solve_all(gpu_ctx, ro, col, w, gid, K)
     for p in range(1, K + 1):
         np.testing.assert_array_equal(got[p - 1], O.run_part(p, ro, col, w, gid, pc))
+
+
+# Graphs with the index's coarse level (32 parts and more), through whole calls and one part a call; two
+# components; directed arcs one way only between regions; a graph without locality keeps the index alone.
+def region_graph(kind):
+    from fastapsp_amd import synth
+    if kind == "grid":
+        u, v, w = synth.grid_graph(72, 72, 0.10, 0.02, 1, 100, 8)
+        return (*synth.to_csr(72 * 72, u, v, w, False), 64)
+    if kind == "large weights":
+        u, v, w = synth.grid_graph(60, 60, 0.10, 0.02, 1, 1 << 23, 9)
+        return (*synth.to_csr(3600, u, v, w, False), 40)
+    if kind == "components":
+        u, v, w = synth.grid_graph(64, 64, 0.05, 0.0, 1, 9, 10)
+        keep = (u // 64 < 30) == (v // 64 < 30)  # the rows below 30 and the others
+        return (*synth.to_csr(4096, u[keep], v[keep], w[keep], False), 48)
+    if kind == "one way":
+        u, v, w = synth.grid_graph(60, 60, 0.05, 0.02, 1, 50, 11)
+        a, b, x = np.concatenate([u, v]), np.concatenate([v, u]), np.concatenate([w, w])
+        keep = (a // 60 < b // 60) | (a // 60 == b // 60) | (a % 7 == 0)  # upwards in every 7th column
+        return (*synth.to_csr(3600, a[keep], b[keep], x[keep], True), 36)
+    return (*random_digraph(2000, 3, 50, 12), 40)  # no locality
+
+
+@pytest.mark.parametrize("kind", ["grid", "large weights", "components", "one way", "no locality"])
+def test_coarse_level(gpu_ctx, kind):
+    import fastapsp_amd as fa
+    ro, col, w, K = region_graph(kind)
+    V = len(ro) - 1
+    with fa.Graph.from_csr(ro, col, w.astype(np.float32), K) as g:
+        g.preCondition()
+        gid = g.getGraphId()
+    got, pc = solve_all(gpu_ctx, ro, col, w, gid, K)
+    for p in range(1, K + 1, 5):
+        np.testing.assert_array_equal(got[p - 1], O.run_part(p, ro, col, w, gid, pc))
+    # one part a call, from a graph whose index is new: the 32nd call makes the coarse level
+    dg = gpu_ctx.upload_graph(ro, col, w)
+    dg.set_partition(gid, pc["st2ed"], pc["ed2st"])
+    sizes = []
+    for p in range(1, K + 1):
+        n, b = int(pc["ver_num"][p]), int(pc["bdy_num"][p])
+        out = gpu_ctx.alloc((n, V))
+        dg.subgraph_solve_batch([int(pc["ver_off"][p])], [n], [b], [out.ptr], V)
+        np.testing.assert_array_equal(out.get(), got[p - 1])
+        out.free()
+        sizes.append(dg.index_info()[1])
+    assert (sizes[30] < sizes[31]) == (kind != "no locality")
+    dg.set_partition(gid, pc["st2ed"], pc["ed2st"])  # drops both
+    assert dg.index_info() == (0, 0)
+    dg.close()

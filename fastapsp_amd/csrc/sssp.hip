@@ -301,6 +301,364 @@ __global__ __launch_bounds__(NF_THREADS) void sssp_nf_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// Few sources (at most two workgroups per CU): a round is a few hundred
+// vertices (512 x 512 grid, band of 8 mean weights: 750 to 930 rounds of 570),
+// and its time is the chain of dependent memory trips and the lines that its
+// gathers touch.  Same words and tags as above, two trips a round, not six:
+//  - the near queues are in LDS, and an entry brings its vertex's arc range
+//    (read beside the relaxation that queues it); entries past the queue's
+//    room, and only they, go through memory;
+//  - four arcs of a vertex come in one step, beside its own word;
+//  - a relaxation is one 64-bit atomic minimum.  Its distance part decides,
+//    and equal distances always carry the same or an older tag: a finite
+//    distance >= threshold has tag ft, the near tag R is the newest, an
+//    unreached word has tag 0.  So a word changes only with its distance, and
+//    the old word that comes back is the one this relaxation improved on, as
+//    with the compare-and-swap.  Rounds of a quarter workgroup and more look
+//    at the words first and leave out what cannot improve: there the trip
+//    costs less than the atomics' lines (256 sources 13.4 -> 8.5 ms);
+//  - a round's barrier waits for LDS only: the words' atomics have returned,
+//    and far-pile entries are not read before a split's own barriers.
+// 512 x 512 grid, before -> now: 74 sources 10.8 -> 6.2 ms, 256 12.7 -> 8.5,
+// 512 (512 threads) 19.2 -> 15.4; 64 x 64 grid, 74 sources 0.81 -> 0.36 ms.  A
+// round of one wave takes 4,600 cycles, one of 1,024 vertices 20,000: there it
+// is bound by the lines its gathers pull through the vector cache (arc ranges
+// read only where needed: same time; unsorted queues: 20% slower).
+typedef int nf_arcs4 __attribute__((ext_vector_type(4), aligned(8)));
+typedef int nf_range __attribute__((ext_vector_type(2), aligned(4)));
+
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Entries of vertex, first and last arc.  One of more than four arcs leaves
+// those past the fourth to an entry of the `rest` list, while that has room:
+// nearly every wave holds such a vertex, and would take a second step, its
+// trips and its instructions, for a lane or two.
+template <int NT>
+struct NearQueues {
+  static constexpr int CAP = 2 * NT, REST = NT / 4;
+  uint32_t v[2][CAP], e[2][CAP], end[2][CAP];
+  uint32_t rv[2][REST], re[2][REST], rend[2][REST];
+
+  __device__ __forceinline__ void put(int b, uint32_t at, uint32_t x, nf_range r) {
+    v[b][at] = x;
+    e[b][at] = (uint32_t)r.x;
+    end[b][at] = (uint32_t)r.y;
+  }
+};
+
+// bin_queue for the n entries of LDS queue b, in place (each thread's two
+// entries wait in registers).
+template <int NT>
+__device__ __forceinline__ void bin_near(NearQueues<NT> &q, int b, uint32_t n, int bsh,
+                                         uint32_t *hist, int *wsum) {
+  constexpr int PER = NBINS / NT;
+  constexpr int NW = NT / 64;
+  static_assert(NearQueues<NT>::CAP == 2 * NT);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+  for (int k = 0; k < PER; k++) hist[tid + k * NT] = 0;
+  uint32_t v[2];
+  nf_range r[2];
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const uint32_t i = tid + k * NT;
+    if (i < n) {
+      v[k] = q.v[b][i];
+      r[k] = nf_range{(int)q.e[b][i], (int)q.end[b][i]};
+    }
+  }
+  lds_barrier();
+#pragma unroll
+  for (int k = 0; k < 2; k++)
+    if (tid + k * NT < n) atomicAdd(&hist[v[k] >> bsh], 1u);
+  lds_barrier();
+  uint32_t loc[PER];
+  uint32_t sum = 0;
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    loc[k] = hist[tid * PER + k];
+    sum += loc[k];
+  }
+  uint32_t x = sum;
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t y = (uint32_t)__shfl_up((int)x, off);
+    if (lane >= off) x += y;
+  }
+  if (lane == 63) wsum[wave] = (int)x;
+  lds_barrier();
+  uint32_t at = x - sum;
+#pragma unroll
+  for (int k = 0; k < NW; k++) at += k < wave ? (uint32_t)wsum[k] : 0u;
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    hist[tid * PER + k] = at;
+    at += loc[k];
+  }
+  lds_barrier();
+#pragma unroll
+  for (int k = 0; k < 2; k++)
+    if (tid + k * NT < n) q.put(b, atomicAdd(&hist[v[k] >> bsh], 1u), v[k], r[k]);
+  lds_barrier();
+}
+
+// This wave's new entries into queue b (near lanes) and at `far`: one LDS
+// atomic makes room for both (counters: near low, far high).  more: memory for
+// the near entries past the queue's room.
+template <int NT, int N>
+__device__ __forceinline__ void wave_put(NearQueues<NT> &q, int b, const bool (&near)[N],
+                                         const bool (&farther)[N], const uint32_t (&v)[N],
+                                         nf_range (&r)[N], unsigned long long *cnt,
+                                         uint32_t *rest, uint32_t *more, uint32_t *far) {
+  using Q = NearQueues<NT>;
+  unsigned long long mn[N], mf[N];
+  uint32_t tn = 0, tf = 0;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    mn[k] = __ballot(near[k]);
+    mf[k] = __ballot(farther[k]);
+    tn += (uint32_t)__popcll(mn[k]);
+    tf += (uint32_t)__popcll(mf[k]);
+  }
+  if (!(tn | tf)) return;
+  unsigned long long base = 0;
+  if (lane_prefix(~0ull) == 0) base = atomicAdd(cnt, ((unsigned long long)tf << 32) | tn);
+  if (tn) {
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const bool big = near[k] && r[k].y - r[k].x > 4;
+      const unsigned long long m = __ballot(big);
+      if (m) {
+        uint32_t at = 0;
+        if (lane_prefix(~0ull) == 0) at = atomicAdd(rest, (uint32_t)__popcll(m));
+        at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) + lane_prefix(m);
+        if (big && at < Q::REST) {
+          q.rv[b][at] = v[k];
+          q.re[b][at] = (uint32_t)r[k].x + 4u;
+          q.rend[b][at] = (uint32_t)r[k].y;
+          r[k].y = r[k].x + 4;
+        }
+      }
+    }
+    uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base);
+    const bool room = at + tn <= Q::CAP;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      if (near[k]) {
+        const uint32_t x = at + lane_prefix(mn[k]);
+        if (room || x < Q::CAP) q.put(b, x, v[k], r[k]);
+        else more[x] = v[k];
+      }
+      at += (uint32_t)__popcll(mn[k]);
+    }
+  }
+  if (tf) {
+    uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(base >> 32));
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      if (farther[k]) far[at + lane_prefix(mf[k])] = v[k];
+      at += (uint32_t)__popcll(mf[k]);
+    }
+  }
+}
+
+template <int NT, bool BIN>
+__global__ __launch_bounds__(NT) void sssp_few_kernel(
+    const int32_t *__restrict__ row_offset, const int2 *__restrict__ edges, int V,
+    const int32_t *__restrict__ sources, int S, int32_t *out, int64_t ld,
+    int32_t *const *__restrict__ rowptr, uint32_t *ws, int64_t ws_stride, int64_t q_off,
+    int delta, int bsh, uint32_t bin_min) {
+  using Q = NearQueues<NT>;
+  __shared__ unsigned long long s_cnt[3];  // near entries low, far entries high
+  __shared__ uint32_t s_rest[3];
+  __shared__ int s_min;
+  __shared__ Q s_q;
+  __shared__ uint32_t s_hist[BIN ? NBINS : 1];
+  __shared__ int s_wsum[BIN ? NT / 64 : 1];
+  uint32_t *base = ws + (int64_t)blockIdx.x * ws_stride;
+  unsigned long long *W = (unsigned long long *)base;  // V words, 8-byte aligned
+  uint32_t *const q0 = base + q_off;
+  const int tid = threadIdx.x;
+  auto word = [&](uint32_t v) {
+    return __hip_atomic_load(W + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  auto range = [&](uint32_t v) { return *reinterpret_cast<const nf_range *>(row_offset + v); };
+  if (tid < 3) {
+    s_cnt[tid] = 0;
+    s_rest[tid] = 0;
+  }
+  int ci = 0;
+  for (int si = blockIdx.x; si < S; si += gridDim.x) {
+    int32_t *dist = rowptr ? rowptr[si] : out + (int64_t)si * ld;
+    const int src = sources[si];
+    for (int v = tid; v < V; v += NT) W[v] = v == src ? nf_word(0, 1u) : nf_word(FAP_INF, 0u);
+    uint32_t *fa = q0 + 2 * (int64_t)V, *fb = q0 + 3 * (int64_t)V;
+    int qb = 1;  // the queue that is filled; the other one is worked on
+    uint32_t n_near = 1, n_rest = 0, n_far = 0;
+    if (tid == 0) s_q.put(0, 0, (uint32_t)src, range(src));
+    uint32_t tags = 2;  // last tag handed out: 1 = the source's, 2 = the first far pile's
+    uint32_t ft = 2;
+    int thr = delta;
+    __syncthreads();
+    // Before the barrier that ends a round or split (counters ci): clears the
+    // next ones.  After it: the new queue.
+    auto clear_next = [&]() {
+      if (tid == 0) {
+        const int cz = ci == 2 ? 0 : ci + 1;
+        s_cnt[cz] = 0;
+        s_rest[cz] = 0;
+      }
+    };
+    auto take = [&]() {
+      const unsigned long long c = s_cnt[ci];
+      const uint32_t nr = s_rest[ci];
+      n_near = (uint32_t)c;
+      n_rest = nr < Q::REST ? nr : Q::REST;
+      ci = ci == 2 ? 0 : ci + 1;
+      // entries past the LDS queue are in memory: everyone's stores first
+      if (n_near > Q::CAP) __syncthreads();
+      qb ^= 1;
+      if constexpr (BIN) {
+        if (n_near >= bin_min && n_near <= Q::CAP)
+          bin_near<NT>(s_q, qb ^ 1, n_near, bsh, s_hist, s_wsum);
+      }
+      return (uint32_t)(c >> 32);
+    };
+    for (;;) {
+      while (n_near > 0) {
+        const uint32_t R = ++tags;
+        const uint32_t n = n_near + n_rest;
+        const bool look = n >= NT / 4;
+        for (uint32_t i0 = 0; i0 < n; i0 += NT) {
+          const uint32_t i = i0 + tid;
+          uint32_t u = 0;
+          int e = 0, end = 0;
+          if (i < n_near) {
+            if (i < Q::CAP) {
+              u = s_q.v[qb ^ 1][i];
+              e = (int)s_q.e[qb ^ 1][i];
+              end = (int)s_q.end[qb ^ 1][i];
+            } else {
+              u = q0[(int64_t)(qb ^ 1) * V + i];
+              const nf_range r = range(u);
+              e = r.x;
+              end = r.y;
+            }
+          } else if (i < n) {
+            u = s_q.rv[qb ^ 1][i - n_near];
+            e = (int)s_q.re[qb ^ 1][i - n_near];
+            end = (int)s_q.rend[qb ^ 1][i - n_near];
+          }
+          while (__any(e < end)) {
+            bool pn[4], pf[4];
+            uint32_t v[4];
+            nf_range r[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+              pn[k] = pf[k] = false;
+              v[k] = 0;
+              r[k] = nf_range{0, 0};
+            }
+            if (e < end) {
+              // four arcs (the array has room for three past its last); those
+              // past the vertex's own repeat the one before, to no effect
+              const nf_arcs4 *p = reinterpret_cast<const nf_arcs4 *>(edges + e);
+              const nf_arcs4 a01 = p[0], a23 = p[1];
+              const int du = nf_dist(word(u));
+              int nd[4];
+              unsigned long long old[4];
+              v[0] = (uint32_t)a01.x;
+              nd[0] = du + a01.y;
+              v[1] = e + 1 < end ? (uint32_t)a01.z : v[0];
+              nd[1] = e + 1 < end ? du + a01.w : nd[0];
+              v[2] = e + 2 < end ? (uint32_t)a23.x : v[1];
+              nd[2] = e + 2 < end ? du + a23.y : nd[1];
+              v[3] = e + 3 < end ? (uint32_t)a23.z : v[2];
+              nd[3] = e + 3 < end ? du + a23.w : nd[2];
+              unsigned long long nw[4];
+#pragma unroll
+              for (int k = 0; k < 4; k++) nw[k] = nf_word(nd[k], nd[k] < thr ? R : ft);
+              if (look) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) old[k] = word(v[k]);
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                  if (nd[k] < nf_dist(old[k])) old[k] = atomicMin(W + v[k], nw[k]);
+              } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++) old[k] = atomicMin(W + v[k], nw[k]);
+              }
+#pragma unroll
+              for (int k = 0; k < 4; k++) r[k] = range(v[k]);
+#pragma unroll
+              for (int k = 0; k < 4; k++) {
+                const bool better = nd[k] < nf_dist(old[k]), near = nd[k] < thr;
+                pn[k] = better && near && (uint32_t)old[k] != R;
+                pf[k] = better && !near && (uint32_t)old[k] != ft;
+              }
+            }
+            wave_put<NT, 4>(s_q, qb, pn, pf, v, r, &s_cnt[ci], &s_rest[ci], q0 + (int64_t)qb * V,
+                            fa + n_far);
+            e += 4;
+          }
+        }
+        clear_next();
+        lds_barrier();
+        n_far += take();
+      }
+      if (n_far == 0) break;
+      // ---- threshold = min live far distance + delta ----
+      if (tid == 0) s_min = 0x7FFFFFFF;
+      __syncthreads();
+      int lmin = 0x7FFFFFFF;
+      for (uint32_t i = tid; i < n_far; i += NT) {
+        const unsigned long long w = word(fa[i]);
+        if ((uint32_t)w == ft) lmin = min(lmin, nf_dist(w));
+      }
+      for (int off = 32; off > 0; off >>= 1) lmin = min(lmin, __shfl_down(lmin, off));
+      if ((tid & 63) == 0) atomicMin(&s_min, lmin);
+      __syncthreads();
+      const int fmin = s_min;
+      if (fmin == 0x7FFFFFFF) break;  // every far entry was stale
+      thr = fmin + delta;
+      const uint32_t rs = ++tags, fn = ++tags;
+      // ---- split the far pile: below thr -> near, else stays far ----
+      for (uint32_t i0 = 0; i0 < n_far; i0 += NT) {
+        const uint32_t i = i0 + tid;
+        bool pn[1] = {false}, pf[1] = {false};
+        uint32_t v[1] = {0};
+        nf_range r[1] = {nf_range{0, 0}};
+        if (i < n_far) {
+          v[0] = fa[i];
+          const unsigned long long w = word(v[0]);
+          r[0] = range(v[0]);
+          if ((uint32_t)w == ft) {
+            const int d = nf_dist(w);
+            pn[0] = d < thr;
+            pf[0] = !pn[0];
+            W[v[0]] = nf_word(d, pn[0] ? rs : fn);
+          }
+        }
+        wave_put<NT, 1>(s_q, qb, pn, pf, v, r, &s_cnt[ci], &s_rest[ci], q0 + (int64_t)qb * V, fb);
+      }
+      ft = fn;
+      clear_next();
+      __syncthreads();
+      n_far = take();
+      uint32_t *t = fa;
+      fa = fb;
+      fb = t;
+    }
+    // every exit follows a barrier, and each thread copies (and the next
+    // source re-initialises) the same words it owns: v = tid mod threads
+    for (int v = tid; v < V; v += NT) dist[v] = nf_dist(word(v));
+  }
+}
+
+// ---------------------------------------------------------------------------
 // In-row state: distances stay below INF = 2^30 - 1, so a vertex's distance
 // and two state bits fit one 32-bit word, d << 2 | state, kept in the output
 // row itself (converted to plain distances in place at the end).  Per-source
@@ -730,12 +1088,25 @@ void launch_group(int grid, hipStream_t s, const fap_graph_dev *g, const int32_t
 template <int NT>
 void launch_single(int grid, hipStream_t s, const fap_graph_dev *g, const int32_t *src,
                    int n_src, int32_t *out, int64_t ld, int32_t *const *rowptr, uint32_t *ws,
-                   int64_t stride, int delta, int bin, int pack, int64_t q_off, int arcs) {
+                   int64_t stride, int delta, int bin, int pack, int64_t q_off, int arcs, bool few) {
   // blocks of 2^bsh vertices, at least 64 (4 lines of distances), at most
   // NBINS blocks; queues of at least bin_min entries are binned
   int bsh = 6;
   while (((int64_t)g->V >> bsh) >= fapk::NBINS) bsh++;
   const uint32_t bin_min = bin >= 3 ? NT / 2 : bin == 2 ? NT : 2 * NT;
+  if constexpr (NT >= 512) {
+    if (pack == 1 && few) {
+      if (bin)
+        hipLaunchKernelGGL((fapk::sssp_few_kernel<NT, true>), dim3(grid), dim3(NT), 0, s,
+                           g->row_offset, g->edges, g->V, src, n_src, out, ld, rowptr, ws, stride,
+                           q_off, delta, bsh, bin_min);
+      else
+        hipLaunchKernelGGL((fapk::sssp_few_kernel<NT, false>), dim3(grid), dim3(NT), 0, s,
+                           g->row_offset, g->edges, g->V, src, n_src, out, ld, rowptr, ws, stride,
+                           q_off, delta, bsh, bin_min);
+      return;
+    }
+  }
   if (pack == 2 && bin)
     hipLaunchKernelGGL((fapk::sssp_nfs_kernel<NT, true>), dim3(grid), dim3(NT), 0, s,
                        g->row_offset, g->edges, g->V, src, n_src, out, ld, rowptr, ws, stride,
@@ -813,10 +1184,14 @@ int run_sssp_rows(fap_ctx *ctx, const fap_graph_dev *g, const int32_t *d_sources
     const int bin = ctx->opt_sssp_bin;
     const int pack = ctx->opt_sssp_pack;
     const int arcs = ctx->opt_sssp_arcs;
+    // as many sources as 512-thread workgroups fit (two a CU); beyond that the
+    // memory system is the limit and both kernels take the same time (1,024
+    // sources of the 512 x 512 grid: 31.7 ms, this one 31.9)
+    const bool few = n_src <= 2 * ctx->num_cus;
     const int64_t q_off = 2 * (((int64_t)V + 63) & ~(int64_t)63);
-    if (threads == 256) launch_single<256>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, delta, bin, pack, q_off, arcs);
-    else if (threads == 512) launch_single<512>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, delta, bin, pack, q_off, arcs);
-    else launch_single<1024>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, delta, bin, pack, q_off, arcs);
+    if (threads == 256) launch_single<256>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, delta, bin, pack, q_off, arcs, few);
+    else if (threads == 512) launch_single<512>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, delta, bin, pack, q_off, arcs, few);
+    else launch_single<1024>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, delta, bin, pack, q_off, arcs, few);
   } else if (group == 4) {
     if (threads == 256) launch_group<4, 256>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, d_off, delta);
     else if (threads == 512) launch_group<4, 512>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, d_off, delta);

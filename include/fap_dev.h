@@ -84,7 +84,9 @@ int fap_ctx_stream(fap_ctx *ctx, void **stream);
  *                           32-bit word of the output row, with a third less
  *                           workspace (2) [1]
  *   "sssp_wgs"     0..8     SSSP workgroups per CU [1024 threads per CU]
- *   "sssp_arcs"    0/1/2/4  arcs each lane relaxes per SSSP step, loads issued together [2]
+ *   "sssp_arcs"    0/1/2/4  arcs each lane relaxes per SSSP step, loads issued together [2];
+ *                           with "sssp_pack" 1, 512 threads or more and at most two
+ *                           sources per CU always 4
  *   "batch_grid"   0..64    batched-closure workgroups per CU per launch [64]
  *   "batch_wait_us" >= 0    longest in-kernel wait of a fap_fw_batched_persistent task
  *                           for its matrix's earlier phases, in microseconds [2 s]

@@ -467,7 +467,7 @@ int fap_graph_upload(fap_ctx *ctx, int32_t V, int64_t E, const int32_t *row_offs
   g->max_degree = maxdeg;
   g->weight_sum = wsum;
   hipError_t e1 = hipMalloc(&g->row_offset, sizeof(int32_t) * (V + 1));
-  hipError_t e2 = hipMalloc(&g->edges, sizeof(int2) * (E + 3));
+  hipError_t e2 = hipMalloc(&g->edges, sizeof(int2) * (E > 0 ? E : 1));
   if (e1 != hipSuccess || e2 != hipSuccess) {
     if (g->row_offset) (void)hipFree(g->row_offset);
     if (g->edges) (void)hipFree(g->edges);

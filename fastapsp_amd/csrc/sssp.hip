@@ -22,13 +22,14 @@
 // Queue appends are compacted per wavefront: a ballot of the pushing lanes,
 // one LDS atomicAdd per wave, lane slot = mbcnt of the ballot.  Duplicates
 // are suppressed by queue state kept beside each distance, in the same word,
-// so an improvement is one compare-and-swap on one cache line (see the two
-// kernels below for the two word layouts).
+// so an improvement is one atomic on one cache line (see the two kernels
+// below for the two word layouts).
 //
 // Every loop is bounded: a vertex enters a queue only after a strict
 // improvement of its distance, and each far split raises the threshold above
 // the smallest far distance.  Workgroups never wait on each other.
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -109,9 +110,9 @@ __device__ __forceinline__ void bin_queue(const uint32_t *__restrict__ q, uint32
 
 // ---------------------------------------------------------------------------
 // Packed state (the default): a vertex's distance and queue tag in one
-// 64-bit word (distance high, tag low), changed together by one
-// compare-and-swap.  A relaxation touches one line of per-source state, not
-// three (distance, round stamp and far tag in separate arrays measured 1.4x
+// 64-bit word (distance high, tag low), changed together by one atomic
+// minimum.  A relaxation touches one line of per-source state, not three
+// (distance, round stamp and far tag in separate arrays measured 1.4x
 // slower), and an improvement costs one atomic instead of two.  The working
 // row belongs to the workgroup; the finished distances are copied to the
 // output row with coalesced stores.
@@ -127,204 +128,41 @@ __device__ __forceinline__ void bin_queue(const uint32_t *__restrict__ q, uint32
 // and the old tag is not this round's R, to the far pile when nd >= threshold
 // and the old tag is not ft.  Distances only decrease and the threshold is
 // fixed between splits, so a vertex is live in the far pile at most once and
-// the split rewrites words with plain stores.  Each failed compare-and-swap
-// means another lane lowered the distance, so the retry loop is bounded.
+// the split rewrites words with plain stores.
+//
+// The minimum of whole words is that of the distances, because equal
+// distances always carry the same or an older tag: a finite distance >=
+// threshold has tag ft, the near tag R is the newest, an unreached word has
+// tag 0.  So a word changes only with its distance, and the old word that
+// comes back is the one this relaxation improved on.
+//
+// A round is a few hundred vertices (512 x 512 grid, band of 8 mean weights:
+// 750 to 930 rounds of 570).  What bounds it: small rounds, the chain of
+// dependent memory trips; larger ones, the vector cache's address rate, about
+// a lane a cycle and CU for gathers (a load more or less per entry in every
+// step: 100 cycles a wave).  So
+//  - the near queues are in LDS, and an entry brings its vertex's arc range;
+//    entries past the queue's room, and only they, go through memory;
+//  - four lanes take an entry, an arc each, so its arcs are one address to
+//    the cache and its own word another; a lane holds one, two or four
+//    entries at a time (a lane with four arcs of one entry: 20% slower at 512
+//    sources);
+//  - a round's barrier waits for LDS only: the words' atomics have returned,
+//    and far-pile entries are not read before a split's own barriers;
+//  - rounds of an eighth of a workgroup and more look at the words first and
+//    leave out what cannot improve, and read the arc ranges of what they
+//    queue alone; below, both go at once with the arcs' own trip saved
+//    (256 sources of the grid with atomics always: 13.4 ms, 8.5 with a look).
+// Measured with a queue in memory, compare-and-swap and a range, arcs, words
+// chain before -> now, 512 x 512 grid: 1 source 9.1 -> 5.0 ms, 74 10.8 ->
+// 5.7, 256 12.7 -> 7.4, 512 19.2 -> 13.0, 3,669 116.9 -> 85.8; 64 x 64 grid:
+// 74 0.81 -> 0.28, 1,024 1.04 -> 0.46.
 __device__ __forceinline__ unsigned long long nf_word(int d, uint32_t tag) {
   return ((unsigned long long)(uint32_t)d << 32) | tag;
 }
 
 __device__ __forceinline__ int nf_dist(unsigned long long w) { return (int)(w >> 32); }
 
-template <int NF_THREADS, bool BIN, int AB>
-__global__ __launch_bounds__(NF_THREADS) void sssp_nf_kernel(
-    const int32_t *__restrict__ row_offset, const int2 *__restrict__ edges, int V,
-    const int32_t *__restrict__ sources, int S, int32_t *out, int64_t ld,
-    int32_t *const *__restrict__ rowptr, uint32_t *ws, int64_t ws_stride, int64_t q_off,
-    int delta, int bsh, uint32_t bin_min) {
-  __shared__ uint32_t s_cnt[6];
-  __shared__ int s_min;
-  __shared__ uint32_t s_hist[BIN ? NBINS : 1];
-  __shared__ int s_wsum[BIN ? NF_THREADS / 64 : 1];
-  uint32_t *base = ws + (int64_t)blockIdx.x * ws_stride;
-  unsigned long long *W = (unsigned long long *)base;  // V words, 8-byte aligned
-  uint32_t *const q0 = base + q_off;
-  const int tid = threadIdx.x;
-  if (tid < 6) s_cnt[tid] = 0;
-  int ci = 0;
-  for (int si = blockIdx.x; si < S; si += gridDim.x) {
-    int32_t *dist = rowptr ? rowptr[si] : out + (int64_t)si * ld;
-    const int src = sources[si];
-    for (int v = tid; v < V; v += NF_THREADS)
-      W[v] = v == src ? nf_word(0, 1u) : nf_word(FAP_INF, 0u);
-    uint32_t *qa = q0, *qb = q0 + V, *fa = q0 + 2 * (int64_t)V, *fb = q0 + 3 * (int64_t)V;
-    uint32_t n_near = 1, n_far = 0;
-    if (tid == 0) qa[0] = (uint32_t)src;
-    uint32_t tags = 2;  // last tag handed out: 1 = the source's, 2 = the first far pile's
-    uint32_t ft = 2;
-    int thr = delta;
-    __syncthreads();
-    for (;;) {
-      while (n_near > 0) {
-        const uint32_t R = ++tags;
-        uint32_t *cn = &s_cnt[2 * ci];
-        for (uint32_t i0 = 0; i0 < n_near; i0 += NF_THREADS) {
-          const uint32_t i = i0 + tid;
-          const bool valid = i < n_near;
-          int du = 0, e = 0, e_end = 0;
-          if (valid) {
-            const int u = (int)qa[i];
-            du = nf_dist(W[u]);
-            e = row_offset[u];
-            e_end = row_offset[u + 1];
-          }
-          // AB arcs per lane per step: their arc and state loads are issued
-          // together, so one step waits for two memory round trips, not 2 AB
-          // (AB = 2 measured 4% faster than 1 and 2% faster than 4)
-          while (__any(valid && e < e_end)) {
-            int2 ed[AB];
-            unsigned long long cur[AB];
-#pragma unroll
-            for (int k = 0; k < AB; k++) {
-              ed[k] = make_int2(0, 0);
-              if (valid && e + k < e_end) ed[k] = edges[e + k];
-            }
-#pragma unroll
-            for (int k = 0; k < AB; k++) {
-              cur[k] = 0;
-              if (valid && e + k < e_end) cur[k] = W[ed[k].x];
-            }
-#pragma unroll
-            for (int k = 0; k < AB; k++) {
-              bool pn = false, pf = false;
-              if (valid && e + k < e_end) {
-                const int nd = du + ed[k].y;
-                unsigned long long *wp = W + ed[k].x;
-                unsigned long long c = cur[k];
-                const bool near = nd < thr;
-                const unsigned long long nw = nf_word(nd, near ? R : ft);
-                while (nd < nf_dist(c)) {
-                  const unsigned long long prev = atomicCAS(wp, c, nw);
-                  if (prev == c) {
-                    const uint32_t old_tag = (uint32_t)c;
-                    if (near) pn = old_tag != R;
-                    else pf = old_tag != ft;
-                    break;
-                  }
-                  c = prev;
-                }
-              }
-              wave_push(pn, (uint32_t)ed[k].x, qb, &cn[0]);
-              wave_push(pf, (uint32_t)ed[k].x, fa + n_far, &cn[1]);
-            }
-            e += AB;
-          }
-        }
-        const int cz = ci == 2 ? 0 : ci + 1;
-        if (tid == 0) {
-          s_cnt[2 * cz] = 0;
-          s_cnt[2 * cz + 1] = 0;
-        }
-        __syncthreads();
-        n_near = cn[0];
-        n_far += cn[1];
-        ci = cz;
-        uint32_t *t = qa;
-        qa = qb;
-        qb = t;
-        if (BIN && n_near >= bin_min) {
-          bin_queue<NF_THREADS>(qa, qb, n_near, bsh, s_hist, s_wsum);
-          t = qa;
-          qa = qb;
-          qb = t;
-        }
-      }
-      if (n_far == 0) break;
-      // ---- threshold = min live far distance + delta ----
-      if (tid == 0) s_min = 0x7FFFFFFF;
-      __syncthreads();
-      int lmin = 0x7FFFFFFF;
-      for (uint32_t i = tid; i < n_far; i += NF_THREADS) {
-        const unsigned long long w = W[fa[i]];
-        if ((uint32_t)w == ft) lmin = min(lmin, nf_dist(w));
-      }
-      for (int off = 32; off > 0; off >>= 1) lmin = min(lmin, __shfl_down(lmin, off));
-      if ((tid & 63) == 0) atomicMin(&s_min, lmin);
-      __syncthreads();
-      const int fmin = s_min;
-      if (fmin == 0x7FFFFFFF) break;  // every far entry was stale
-      thr = fmin + delta;
-      const uint32_t rs = ++tags, fn = ++tags;
-      // ---- split the far pile: below thr -> near, else stays far ----
-      uint32_t *cn = &s_cnt[2 * ci];
-      for (uint32_t i0 = 0; i0 < n_far; i0 += NF_THREADS) {
-        const uint32_t i = i0 + tid;
-        bool pn = false, pf = false;
-        uint32_t item = 0;
-        if (i < n_far) {
-          const int v = (int)fa[i];
-          item = (uint32_t)v;
-          const unsigned long long w = W[v];
-          if ((uint32_t)w == ft) {
-            const int d = nf_dist(w);
-            pn = d < thr;
-            pf = !pn;
-            W[v] = nf_word(d, pn ? rs : fn);
-          }
-        }
-        wave_push(pn, item, qa, &cn[0]);
-        wave_push(pf, item, fb, &cn[1]);
-      }
-      ft = fn;
-      const int cz = ci == 2 ? 0 : ci + 1;
-      if (tid == 0) {
-        s_cnt[2 * cz] = 0;
-        s_cnt[2 * cz + 1] = 0;
-      }
-      __syncthreads();
-      n_near = cn[0];
-      n_far = cn[1];
-      ci = cz;
-      uint32_t *t = fa;
-      fa = fb;
-      fb = t;
-      if (BIN && n_near >= bin_min) {
-        bin_queue<NF_THREADS>(qa, qb, n_near, bsh, s_hist, s_wsum);
-        t = qa;
-        qa = qb;
-        qb = t;
-      }
-    }
-    // every exit follows a barrier, and each thread copies (and the next
-    // source re-initialises) the same words it owns: v = tid mod threads
-    for (int v = tid; v < V; v += NF_THREADS) dist[v] = nf_dist(W[v]);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Few sources (at most two workgroups per CU): a round is a few hundred
-// vertices (512 x 512 grid, band of 8 mean weights: 750 to 930 rounds of 570),
-// and its time is the chain of dependent memory trips and the lines that its
-// gathers touch.  Same words and tags as above, two trips a round, not six:
-//  - the near queues are in LDS, and an entry brings its vertex's arc range
-//    (read beside the relaxation that queues it); entries past the queue's
-//    room, and only they, go through memory;
-//  - four arcs of a vertex come in one step, beside its own word;
-//  - a relaxation is one 64-bit atomic minimum.  Its distance part decides,
-//    and equal distances always carry the same or an older tag: a finite
-//    distance >= threshold has tag ft, the near tag R is the newest, an
-//    unreached word has tag 0.  So a word changes only with its distance, and
-//    the old word that comes back is the one this relaxation improved on, as
-//    with the compare-and-swap.  Rounds of a quarter workgroup and more look
-//    at the words first and leave out what cannot improve: there the trip
-//    costs less than the atomics' lines (256 sources 13.4 -> 8.5 ms);
-//  - a round's barrier waits for LDS only: the words' atomics have returned,
-//    and far-pile entries are not read before a split's own barriers.
-// 512 x 512 grid, before -> now: 74 sources 10.8 -> 6.2 ms, 256 12.7 -> 8.5,
-// 512 (512 threads) 19.2 -> 15.4; 64 x 64 grid, 74 sources 0.81 -> 0.36 ms.  A
-// round of one wave takes 4,600 cycles, one of 1,024 vertices 20,000: there it
-// is bound by the lines its gathers pull through the vector cache (arc ranges
-// read only where needed: same time; unsorted queues: 20% slower).
-typedef int nf_arcs4 __attribute__((ext_vector_type(4), aligned(8)));
 typedef int nf_range __attribute__((ext_vector_type(2), aligned(4)));
 
 __device__ __forceinline__ void lds_barrier() {
@@ -466,7 +304,7 @@ __device__ __forceinline__ void wave_put(NearQueues<NT> &q, int b, const bool (&
 }
 
 template <int NT, bool BIN>
-__global__ __launch_bounds__(NT) void sssp_few_kernel(
+__global__ __launch_bounds__(NT) void sssp_nf_kernel(
     const int32_t *__restrict__ row_offset, const int2 *__restrict__ edges, int V,
     const int32_t *__restrict__ sources, int S, int32_t *out, int64_t ld,
     int32_t *const *__restrict__ rowptr, uint32_t *ws, int64_t ws_stride, int64_t q_off,
@@ -531,78 +369,102 @@ __global__ __launch_bounds__(NT) void sssp_few_kernel(
       while (n_near > 0) {
         const uint32_t R = ++tags;
         const uint32_t n = n_near + n_rest;
-        const bool look = n >= NT / 4;
-        for (uint32_t i0 = 0; i0 < n; i0 += NT) {
-          const uint32_t i = i0 + tid;
-          uint32_t u = 0;
-          int e = 0, end = 0;
-          if (i < n_near) {
-            if (i < Q::CAP) {
-              u = s_q.v[qb ^ 1][i];
-              e = (int)s_q.e[qb ^ 1][i];
-              end = (int)s_q.end[qb ^ 1][i];
-            } else {
-              u = q0[(int64_t)(qb ^ 1) * V + i];
-              const nf_range r = range(u);
-              e = r.x;
-              end = r.y;
-            }
-          } else if (i < n) {
-            u = s_q.rv[qb ^ 1][i - n_near];
-            e = (int)s_q.re[qb ^ 1][i - n_near];
-            end = (int)s_q.rend[qb ^ 1][i - n_near];
-          }
-          while (__any(e < end)) {
-            bool pn[4], pf[4];
-            uint32_t v[4];
-            nf_range r[4];
+        const bool look = n >= NT / 8;
+        // four lanes to an entry, an arc each; a lane takes part in N entries,
+        // NT / 4 apart
+        auto relax = [&](auto width, uint32_t i0) {
+          constexpr int N = decltype(width)::value;
+          uint32_t u[N];
+          int e[N], end[N];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-              pn[k] = pf[k] = false;
-              v[k] = 0;
-              r[k] = nf_range{0, 0};
-            }
-            if (e < end) {
-              // four arcs (the array has room for three past its last); those
-              // past the vertex's own repeat the one before, to no effect
-              const nf_arcs4 *p = reinterpret_cast<const nf_arcs4 *>(edges + e);
-              const nf_arcs4 a01 = p[0], a23 = p[1];
-              const int du = nf_dist(word(u));
-              int nd[4];
-              unsigned long long old[4];
-              v[0] = (uint32_t)a01.x;
-              nd[0] = du + a01.y;
-              v[1] = e + 1 < end ? (uint32_t)a01.z : v[0];
-              nd[1] = e + 1 < end ? du + a01.w : nd[0];
-              v[2] = e + 2 < end ? (uint32_t)a23.x : v[1];
-              nd[2] = e + 2 < end ? du + a23.y : nd[1];
-              v[3] = e + 3 < end ? (uint32_t)a23.z : v[2];
-              nd[3] = e + 3 < end ? du + a23.w : nd[2];
-              unsigned long long nw[4];
-#pragma unroll
-              for (int k = 0; k < 4; k++) nw[k] = nf_word(nd[k], nd[k] < thr ? R : ft);
-              if (look) {
-#pragma unroll
-                for (int k = 0; k < 4; k++) old[k] = word(v[k]);
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-                  if (nd[k] < nf_dist(old[k])) old[k] = atomicMin(W + v[k], nw[k]);
+          for (int k = 0; k < N; k++) {
+            const uint32_t i = i0 + k * (NT / 4) + (tid >> 2);
+            u[k] = 0;
+            e[k] = end[k] = 0;
+            if (i < n_near) {
+              if (i < Q::CAP) {
+                u[k] = s_q.v[qb ^ 1][i];
+                e[k] = (int)s_q.e[qb ^ 1][i];
+                end[k] = (int)s_q.end[qb ^ 1][i];
               } else {
-#pragma unroll
-                for (int k = 0; k < 4; k++) old[k] = atomicMin(W + v[k], nw[k]);
+                u[k] = q0[(int64_t)(qb ^ 1) * V + i];
+                const nf_range r = range(u[k]);
+                e[k] = r.x;
+                end[k] = r.y;
               }
-#pragma unroll
-              for (int k = 0; k < 4; k++) r[k] = range(v[k]);
-#pragma unroll
-              for (int k = 0; k < 4; k++) {
-                const bool better = nd[k] < nf_dist(old[k]), near = nd[k] < thr;
-                pn[k] = better && near && (uint32_t)old[k] != R;
-                pf[k] = better && !near && (uint32_t)old[k] != ft;
-              }
+            } else if (i < n) {
+              u[k] = s_q.rv[qb ^ 1][i - n_near];
+              e[k] = (int)s_q.re[qb ^ 1][i - n_near];
+              end[k] = (int)s_q.rend[qb ^ 1][i - n_near];
             }
-            wave_put<NT, 4>(s_q, qb, pn, pf, v, r, &s_cnt[ci], &s_rest[ci], q0 + (int64_t)qb * V,
+            e[k] += tid & 3;
+          }
+          for (;;) {
+            bool more = false;
+#pragma unroll
+            for (int k = 0; k < N; k++) more |= e[k] < end[k];
+            if (!__any(more)) break;
+            bool act[N], pn[N], pf[N];
+            uint32_t v[N];
+            nf_range r[N];
+            int2 arc[N];
+            int nd[N];
+            unsigned long long old[N], nw[N];
+            // lanes without an arc read the first one, and no word but word 0
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+              act[k] = e[k] < end[k];
+              arc[k] = edges[act[k] ? e[k] : 0];
+              old[k] = word(u[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+              v[k] = act[k] ? (uint32_t)arc[k].x : 0u;
+              nd[k] = act[k] ? nf_dist(old[k]) + arc[k].y : 0x7FFFFFFF;
+              nw[k] = nf_word(nd[k], nd[k] < thr ? R : ft);
+            }
+            if (look) {
+#pragma unroll
+              for (int k = 0; k < N; k++) old[k] = word(v[k]);
+#pragma unroll
+              for (int k = 0; k < N; k++)
+                if (nd[k] < nf_dist(old[k])) old[k] = atomicMin(W + v[k], nw[k]);
+            } else {
+#pragma unroll
+              for (int k = 0; k < N; k++) {
+                old[k] = 0;
+                if (act[k]) old[k] = atomicMin(W + v[k], nw[k]);
+              }
+#pragma unroll
+              for (int k = 0; k < N; k++) r[k] = range(v[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+              const bool better = nd[k] < nf_dist(old[k]), near = nd[k] < thr;
+              pn[k] = better && near && (uint32_t)old[k] != R;
+              pf[k] = better && !near && (uint32_t)old[k] != ft;
+            }
+            if (look) {
+#pragma unroll
+              for (int k = 0; k < N; k++)
+                if (pn[k]) r[k] = range(v[k]);
+            }
+            wave_put<NT, N>(s_q, qb, pn, pf, v, r, &s_cnt[ci], &s_rest[ci], q0 + (int64_t)qb * V,
                             fa + n_far);
-            e += 4;
+#pragma unroll
+            for (int k = 0; k < N; k++) e[k] += 4;
+          }
+        };
+        for (uint32_t i0 = 0; i0 < n;) {
+          if (n - i0 <= NT / 4) {
+            relax(std::integral_constant<int, 1>(), i0);
+            i0 += NT / 4;
+          } else if (n - i0 <= NT / 2) {
+            relax(std::integral_constant<int, 2>(), i0);
+            i0 += NT / 2;
+          } else {
+            relax(std::integral_constant<int, 4>(), i0);
+            i0 += NT;
           }
         }
         clear_next();
@@ -1088,25 +950,12 @@ void launch_group(int grid, hipStream_t s, const fap_graph_dev *g, const int32_t
 template <int NT>
 void launch_single(int grid, hipStream_t s, const fap_graph_dev *g, const int32_t *src,
                    int n_src, int32_t *out, int64_t ld, int32_t *const *rowptr, uint32_t *ws,
-                   int64_t stride, int delta, int bin, int pack, int64_t q_off, int arcs, bool few) {
+                   int64_t stride, int delta, int bin, int pack, int64_t q_off) {
   // blocks of 2^bsh vertices, at least 64 (4 lines of distances), at most
   // NBINS blocks; queues of at least bin_min entries are binned
   int bsh = 6;
   while (((int64_t)g->V >> bsh) >= fapk::NBINS) bsh++;
   const uint32_t bin_min = bin >= 3 ? NT / 2 : bin == 2 ? NT : 2 * NT;
-  if constexpr (NT >= 512) {
-    if (pack == 1 && few) {
-      if (bin)
-        hipLaunchKernelGGL((fapk::sssp_few_kernel<NT, true>), dim3(grid), dim3(NT), 0, s,
-                           g->row_offset, g->edges, g->V, src, n_src, out, ld, rowptr, ws, stride,
-                           q_off, delta, bsh, bin_min);
-      else
-        hipLaunchKernelGGL((fapk::sssp_few_kernel<NT, false>), dim3(grid), dim3(NT), 0, s,
-                           g->row_offset, g->edges, g->V, src, n_src, out, ld, rowptr, ws, stride,
-                           q_off, delta, bsh, bin_min);
-      return;
-    }
-  }
   if (pack == 2 && bin)
     hipLaunchKernelGGL((fapk::sssp_nfs_kernel<NT, true>), dim3(grid), dim3(NT), 0, s,
                        g->row_offset, g->edges, g->V, src, n_src, out, ld, rowptr, ws, stride,
@@ -1115,20 +964,12 @@ void launch_single(int grid, hipStream_t s, const fap_graph_dev *g, const int32_
     hipLaunchKernelGGL((fapk::sssp_nfs_kernel<NT, false>), dim3(grid), dim3(NT), 0, s,
                        g->row_offset, g->edges, g->V, src, n_src, out, ld, rowptr, ws, stride,
                        delta, bsh, bin_min);
-  else if (bin && arcs == 4)
-    hipLaunchKernelGGL((fapk::sssp_nf_kernel<NT, true, 4>), dim3(grid), dim3(NT), 0, s,
-                       g->row_offset, g->edges, g->V, src, n_src, out, ld, rowptr, ws, stride,
-                       q_off, delta, bsh, bin_min);
-  else if (bin && arcs == 2)
-    hipLaunchKernelGGL((fapk::sssp_nf_kernel<NT, true, 2>), dim3(grid), dim3(NT), 0, s,
-                       g->row_offset, g->edges, g->V, src, n_src, out, ld, rowptr, ws, stride,
-                       q_off, delta, bsh, bin_min);
   else if (bin)
-    hipLaunchKernelGGL((fapk::sssp_nf_kernel<NT, true, 1>), dim3(grid), dim3(NT), 0, s,
+    hipLaunchKernelGGL((fapk::sssp_nf_kernel<NT, true>), dim3(grid), dim3(NT), 0, s,
                        g->row_offset, g->edges, g->V, src, n_src, out, ld, rowptr, ws, stride,
                        q_off, delta, bsh, bin_min);
   else
-    hipLaunchKernelGGL((fapk::sssp_nf_kernel<NT, false, 2>), dim3(grid), dim3(NT), 0, s,
+    hipLaunchKernelGGL((fapk::sssp_nf_kernel<NT, false>), dim3(grid), dim3(NT), 0, s,
                        g->row_offset, g->edges, g->V, src, n_src, out, ld, rowptr, ws, stride,
                        q_off, delta, bsh, bin_min);
 }
@@ -1183,15 +1024,10 @@ int run_sssp_rows(fap_ctx *ctx, const fap_graph_dev *g, const int32_t *d_sources
     // state words first (V of 8 bytes), then the four queues
     const int bin = ctx->opt_sssp_bin;
     const int pack = ctx->opt_sssp_pack;
-    const int arcs = ctx->opt_sssp_arcs;
-    // as many sources as 512-thread workgroups fit (two a CU); beyond that the
-    // memory system is the limit and both kernels take the same time (1,024
-    // sources of the 512 x 512 grid: 31.7 ms, this one 31.9)
-    const bool few = n_src <= 2 * ctx->num_cus;
     const int64_t q_off = 2 * (((int64_t)V + 63) & ~(int64_t)63);
-    if (threads == 256) launch_single<256>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, delta, bin, pack, q_off, arcs, few);
-    else if (threads == 512) launch_single<512>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, delta, bin, pack, q_off, arcs, few);
-    else launch_single<1024>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, delta, bin, pack, q_off, arcs, few);
+    if (threads == 256) launch_single<256>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, delta, bin, pack, q_off);
+    else if (threads == 512) launch_single<512>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, delta, bin, pack, q_off);
+    else launch_single<1024>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, delta, bin, pack, q_off);
   } else if (group == 4) {
     if (threads == 256) launch_group<4, 256>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, d_off, delta);
     else if (threads == 512) launch_group<4, 512>(grid, s, g, src, n_src, d_out, ld_out, d_rowptr, ws, stride, d_off, delta);

@@ -96,12 +96,18 @@ void sssp_settings(const fap_ctx *ctx, const fap_graph_dev *g, int32_t n_src, in
   // sources fit on the CUs, smaller workgroups (more per CU) beyond, and a
   // band that narrows as more sources run at once (fewer re-relaxations
   // where the memory system is the limit, fewer rounds where it is not).
-  // Measured on the 512x512 grid: 74 sources 10.2 ms at 1024 threads vs
-  // 18.2 ms at 256, band 8 x mean weight best (10.9 ms at 4 x); 3669
-  // sources 119 ms at 256 threads vs 165 ms at 1024, band 3-4 x best
-  // (110 ms, 120 ms at 8 x).
+  // Beyond two sources a CU, many vertices want 512 threads: fronts that fill
+  // them, and half as many 8 V byte states at a time share the caches.
+  // Measured on grids: 512 x 512, 256 sources 7.4 ms at 1024 threads, 7.8 at
+  // 512; 512 sources 13.0 at 512 threads, 14.3 at 1024, 15.2 at 256; 3,669
+  // sources 85.8 at 512 threads, 98.6 at 256; 256 x 256, 3,669 sources 21.0
+  // and 19.8; 64 x 64, 1,024 sources 0.68 and 0.46.  Band, in mean weights:
+  // 74 sources 5.55 ms at 4, 5.71 at 8 (64 x 64: 0.32, 0.28); 1,024 sources
+  // 24.4 at 4, 25.8 at 6, 24.9 at 2.
   const int cus = ctx ? ctx->num_cus : 256;
-  const int by_count = n_src <= cus ? 1024 : n_src <= 2 * cus ? 512 : 256;
+  const int by_count = n_src <= cus                             ? 1024
+                       : n_src <= 2 * cus || g->V >= (1 << 17) ? 512
+                                                                : 256;
   const double mult_by_count = n_src <= cus ? 8.0 : n_src <= 2 * cus ? 6.0 : 4.0;
   *threads = (ctx && ctx->opt_sssp_threads > 0) ? ctx->opt_sssp_threads : cached ? p[0] : by_count;
   // Grouped sources only on request: on the same grid a group of 8 takes

@@ -72,7 +72,8 @@ int fap_ctx_stream(fap_ctx *ctx, void **stream);
  *   "fw_lookahead" -1/0/1   overlap FW round r+1's diagonal/panels with round r [0]
  *   "fw_tile"      0/64/128 FW block size [64]
  *   "sssp_threads" 0/256/512/1024  threads per SSSP workgroup [1024 while the sources
- *                           fit on the CUs, 512 up to twice that, 256 beyond]
+ *                           fit on the CUs, 512 up to twice that, beyond that 256, or
+ *                           512 for graphs of 2^17 vertices and more]
  *   "sssp_delta"   >= 0     near-far band width [graph's own, else 8 / 6 / 4 x mean
  *                           weight for sources up to the CU count / twice it / more]
  *   "sssp_group"   0/1/4/8  sources per SSSP workgroup pass [1]
@@ -84,9 +85,7 @@ int fap_ctx_stream(fap_ctx *ctx, void **stream);
  *                           32-bit word of the output row, with a third less
  *                           workspace (2) [1]
  *   "sssp_wgs"     0..8     SSSP workgroups per CU [1024 threads per CU]
- *   "sssp_arcs"    0/1/2/4  arcs each lane relaxes per SSSP step, loads issued together [2];
- *                           with "sssp_pack" 1, 512 threads or more and at most two
- *                           sources per CU always 4
+ *   "sssp_arcs"    0/1/2/4  accepted; an SSSP step takes four arcs of a vertex at once [2]
  *   "batch_grid"   0..64    batched-closure workgroups per CU per launch [64]
  *   "batch_wait_us" >= 0    longest in-kernel wait of a fap_fw_batched_persistent task
  *                           for its matrix's earlier phases, in microseconds [2 s]

@@ -20,7 +20,8 @@
  *
  * With no entry the defaults are tile 128 when ceil(n / 128) - 1 squared is
  * at least 8 per CU (64 below), no look-ahead, SSSP threads 1024
- * while the sources fit on the CUs (512 up to twice that, 256 beyond),
+ * while the sources fit on the CUs (512 up to twice that, beyond it 256, or 512 from
+ * 2^17 vertices),
  * delta 8 x mean weight while the sources fit on the CUs (6 x up to twice
  * that, 4 x beyond), 64 workgroups per CU.
  *

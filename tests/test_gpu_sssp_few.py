@@ -1,4 +1,4 @@
-"""Few-source SSSP kernel: LDS queues and their ends (GPU), against Dijkstra.
+"""SSSP kernel: LDS queues and their ends (GPU), against Dijkstra.
 
 The kernel keeps the near queue of a workgroup of NT threads in LDS (2 NT
 entries, later ones in memory) and the arcs past a vertex's fourth in a second
@@ -35,7 +35,8 @@ def graph(kind):
 
 
 @pytest.mark.parametrize("kind", ["star", "dense", "wide", "heavy", "single", "grid"])
-@pytest.mark.parametrize("threads,delta,binq", [(1024, 0, 3), (512, 1, 3), (512, 1 << 24, 0)])
+@pytest.mark.parametrize("threads,delta,binq", [(1024, 0, 3), (512, 1, 3), (512, 1 << 24, 0),
+                                                (256, 0, 3)])
 def test_few_sources(gpu_ctx, kind, threads, delta, binq):
     V, u, v, w, directed = graph(kind)
     keep = u != v

@@ -9,12 +9,12 @@
 //   2. row panel (r, J) = min(C, D_rr (x) C) and column panel
 //      (I, r) = min(C, C (x) D_rr) for all I, J != r: one launch;
 //   3. every other tile (I, J) = min(C, D_Ir (x) D_rJ): one launch.
-// Phases 2 and 3 reuse the register-blocked min-plus tile (minplus_tile.h)
-// with T x T tiles; phase 3 of T = 128 runs its additions on the matrix cores
-// (mfma_tile.h).  T = 128 halves the number of rounds and, with 8 x 8
-// cells per lane, the LDS bytes per update (phase 3 is bound by LDS reads
-// at 4 x 4 cells); T = 64 gives 4x more tiles per launch and a cheap
-// diagonal phase.  128 is the default for large n, 64 below (launch_fw).
+// Phases 2 and 3 run T x T tiles with their additions on the matrix cores
+// (mfma_tile.h; the panels of T = 128 in 64 x 64 quarters on the VALU).
+// T = 128 halves the number of rounds and the passes over the matrix, which
+// bound phase 3 (T = 64, n = 3800: 116 MB in 38 us, 19 us of arithmetic);
+// T = 64 has a cheaper chain of diagonal and panels.  128 is the default for
+// large n, 64 below (launch_fw).
 #include <type_traits>
 
 #include "common.h"
@@ -145,11 +145,13 @@ __global__ __launch_bounds__(FW_DIAG_THREADS) void fw_round_kernel(int32_t *d, i
 
 // Phase 2: workgroups [0, nb-1) take row-panel tiles (r, J), the next nb-1
 // take column-panel tiles (I, r).  Each tile is owned by one workgroup and
-// aliases one operand; the tile reads all operands before writing C.
+// aliases one operand; the tile reads all operands before writing C.  On the
+// matrix-core tile, as phase 3, for any alignment (n = 2999 at an odd row
+// stride 2.95 -> 2.01 ms with both; the 4 x 4 integer tile before).
 template <int TM>
 __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void fw_panel_kernel(
     int32_t *d, int n, int64_t ld, int r, int nb, int flags) {
-  using Tile = MpTile<TM, TM>;
+  using Tile = MxSmall;
   constexpr int T = Tile::BM;
   __shared__ __attribute__((aligned(16))) int32_t lds[Tile::LDS_WORDS];
   const int base = r * T;
@@ -221,7 +223,7 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(8)))
 template <int TM, bool fuse>
 __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void fw_rest_kernel(
     int32_t *d, int n, int64_t ld, int r, int nb, int flags, int mode) {
-  using Tile = typename std::conditional<TM == 8, MxBig, MpTile<TM, TM>>::type;
+  using Tile = typename std::conditional<TM == 8, MxBig, MxSmall>::type;
   constexpr int T = Tile::BM;
   constexpr int CLOSE_WORDS = TM == 4 ? CLOSE64_WORDS : CLOSE128_WORDS;
   constexpr int LDS_WORDS = CLOSE_WORDS > Tile::LDS_WORDS ? CLOSE_WORDS : Tile::LDS_WORDS;
@@ -328,11 +330,12 @@ struct Fw {
     const int flags = vec_flags(d, ld, d, ld, d, ld);
     FAP_TRY(diag_panel(d, n, ld, 0, nb, flags, s));
     const bool overlap = lookahead && ctx && ctx->aux_stream && nb >= 3;
-    // fuse the next diagonal closure into phase 3 when the phase is long
-    // enough to hide it: at least 8 tiles per CU for T = 64 (a 256-thread
-    // 64-closure), 4 for T = 128 (the 128-closure's seven steps)
+    // phase 3 also closes the next diagonal block, beside its other tiles,
+    // from one tile per CU on: no launch for it, and it starts a phase early
+    // (T = 64: n = 1250 0.73 -> 0.62 ms, 2048 1.13 -> 0.94, 2560 -> 1.22;
+    // T = 128: 4096 3.89 -> 3.67)
     const int64_t cus = ctx ? ctx->num_cus : 256;
-    const bool fuse_ok = (int64_t)(nb - 1) * (nb - 1) >= cus * (TM == 4 ? 8 : 4);
+    const bool fuse_ok = (int64_t)(nb - 1) * (nb - 1) >= cus;
     for (int r = 0; r < nb; r++) {
       if (r + 1 < nb && overlap) {
         FAP_TRY(rest(d, n, ld, r, nb, flags, 1, s));
@@ -343,10 +346,6 @@ struct Fw {
         FAP_TRY(rest(d, n, ld, r, nb, flags, 2, s));
         FAP_HIP(hipStreamWaitEvent(s, ctx->ev_fw_panel, 0));
       } else {
-        // round r's phase 3 also closes the next diagonal block when the
-        // phase is long enough to hide it (below that the 1024-thread
-        // diagonal kernel is faster: T = 64, n = 1024 took 0.56 ms unfused,
-        // 0.64 ms fused)
         const int fuse = (fuse_ok && r + 1 < nb) ? 1 : 0;
         FAP_TRY(rest(d, n, ld, r, nb, flags, 0, s, fuse));
         if (r + 1 < nb) FAP_TRY(diag_panel(d, n, ld, r + 1, nb, flags, s, !fuse));

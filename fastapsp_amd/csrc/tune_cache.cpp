@@ -75,11 +75,12 @@ fap_tune_cache *tune_env_cache() {
 void fw_settings(const fap_ctx *ctx, int32_t n, int *tile, bool *lookahead) {
   int32_t p[2] = {64, 0};
   const bool cached = tune_lookup(ctx, "fw", fap_tune_key_fw(n), p);
-  // default: 128 once phase 3 has at least 8 tiles of 128 x 128 per CU
-  // (n >= ~6,000 on 256 CUs), where it measured faster; 64 below
+  // default: 128 once phase 3 has at least 4 tiles of 128 x 128 per CU (n >=
+  // 4225 on 256 CUs), where it measured faster (4096: 3.67 ms, 3.37 at 64;
+  // 4500: 4.20 and 4.69); 64 below
   const int64_t nb128 = ((int64_t)n + 127) / 128;
   const int def_tile =
-      (nb128 - 1) * (nb128 - 1) >= 8 * (int64_t)(ctx ? ctx->num_cus : 256) ? 128 : 64;
+      (nb128 - 1) * (nb128 - 1) >= 4 * (int64_t)(ctx ? ctx->num_cus : 256) ? 128 : 64;
   *tile = (ctx && (ctx->opt_fw_tile == 64 || ctx->opt_fw_tile == 128)) ? ctx->opt_fw_tile
           : cached                                                     ? p[0]
                                                                        : def_tile;

@@ -149,7 +149,7 @@ __global__ __launch_bounds__(FW_DIAG_THREADS) void fw_round_kernel(int32_t *d, i
 // matrix-core tile, as phase 3, for any alignment (n = 2999 at an odd row
 // stride 2.95 -> 2.01 ms with both; the 4 x 4 integer tile before).
 template <int TM>
-__global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void fw_panel_kernel(
+__global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6))) void fw_panel_kernel(
     int32_t *d, int n, int64_t ld, int r, int nb, int flags) {
   using Tile = MxSmall;
   constexpr int T = Tile::BM;
@@ -219,9 +219,10 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(8)))
 // swapping with the workgroup that had it -- and after its update closes
 // it (in LDS for T = 64, by close_block128 for T = 128): the next round's
 // diagonal phase, done while the other tiles of this phase run, so that
-// round launches only its panels.
+// round launches only its panels.  T = 64 wants 6 waves per SIMD (77 VGPRs, no
+// call inside): n = 3500 2.58 ms, 2.73 at the 4 that its callees would leave.
 template <int TM, bool fuse>
-__global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void fw_rest_kernel(
+__global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(TM == 4 ? 6 : 4, TM == 4 ? 6 : 4))) void fw_rest_kernel(
     int32_t *d, int n, int64_t ld, int r, int nb, int flags, int mode) {
   using Tile = typename std::conditional<TM == 8, MxBig, MxSmall>::type;
   constexpr int T = Tile::BM;
@@ -268,7 +269,7 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
   Tile::run(a, ld, b, ld, c, ld, imin(T, n - I * T), imin(T, n - J * T), kb, true, flags, lds);
   if (fuse && blockIdx.x == 0) {
     __syncthreads();  // the tile's writes above come before the closure reads it
-    if (T == 64) close_block64_call<4>((mp_out_ptr)c, ld, imin(T, n - I * T), (mp_lds_ptr)lds);
+    if constexpr (T == 64) close_block64<4>(c, ld, imin(T, n - I * T), lds);
     else close_block128_call((mp_out_ptr)c, ld, imin(T, n - I * T), (mp_lds_ptr)lds);
   }
 }

@@ -248,8 +248,13 @@ struct MxTile {
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[i][j][r] = 0x7F800000;  // above every sum: INF
     if (!fits(lda, ldb, n_valid, K) || product(A, lda, B, ldb, m_valid, n_valid, K, lds, acc)) {
-      int_tile<NI, NJ>((mp_in_ptr)A, lda, (mp_in_ptr)B, ldb, (mp_out_ptr)C, ldc, m_valid, n_valid,
-                       K, accumulate, flags, (mp_lds_ptr)lds);
+      if constexpr (NI * NJ == 1) {  // small enough in place, at 6 waves per SIMD
+        __syncthreads();
+        MpTile<4, 4>::run(A, lda, B, ldb, C, ldc, m_valid, n_valid, K, accumulate, flags, lds);
+      } else {
+        int_tile<NI, NJ>((mp_in_ptr)A, lda, (mp_in_ptr)B, ldb, (mp_out_ptr)C, ldc, m_valid,
+                         n_valid, K, accumulate, flags, (mp_lds_ptr)lds);
+      }
       return;
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;

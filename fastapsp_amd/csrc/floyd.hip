@@ -370,7 +370,7 @@ static int run_rounds(int32_t *d, int32_t n, int64_t ld, hipStream_t s) {
 }
 
 // Block size and look-ahead: the context options if set, else the tune
-// cache, else 128 when phase 3 has at least 8 tiles of 128 per CU and 64
+// cache, else 128 when phase 3 has at least 4 tiles of 128 per CU and 64
 // below, without look-ahead (fw_settings).  Measured on MI355X (closure
 // ms, T = 64 / 128): n = 8192 20.7 / 19.0, 6144 9.49 / 8.86, 5120 5.99 /
 // 6.54, 4096 3.59 / 4.87, 2048 1.40 / 1.83 -- the 128 x 128 tile with 8 x 8
@@ -384,12 +384,12 @@ int launch_fw(fap_ctx *ctx, int32_t *d, int32_t n, int64_t ld, hipStream_t s) {
   bool lookahead;
   fw_settings(ctx, n, &tile, &lookahead);
   if (tile == 128) return Fw<8>::run(ctx, d, n, ld, lookahead, s);
-  // Up to 1.5 workgroups per CU a round in one launch wins although every
-  // workgroup closes the pivot block and makes its own panel tile (closure us,
-  // one / three launches a round: n = 97 44 / 66, 512 160 / 243, 1024 331 /
-  // 494, 1200 579 / 662; 1448 1021 / 829: two full workgroups per CU).
+  // Up to a workgroup per CU a round in one launch wins although every
+  // workgroup closes the pivot block and makes its own panel tile (us, a
+  // launch a round / phases: n = 97 44 / 66, 512 160 / 243, 900 346 / 483,
+  // 1024 325 / 470; past it 1088 484 / 465, 1216 546 / 527).
   const int64_t nb = (n + 63) / 64;
-  if (!lookahead && 2 * nb * nb <= 3 * (int64_t)(ctx ? ctx->num_cus : 256))
+  if (!lookahead && nb * nb <= (int64_t)(ctx ? ctx->num_cus : 256))
     return run_rounds(d, n, ld, s);
   return Fw<4>::run(ctx, d, n, ld, lookahead, s);
 }

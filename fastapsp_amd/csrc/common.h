@@ -66,6 +66,7 @@ struct fap_graph_dev {
   int32_t delta = 0;  // SSSP near-far band width (0 = derived from the mean weight)
   int32_t *in_offset = nullptr;  // transposed CSR (V+1), built on first path request
   int2 *in_arcs = nullptr;       // E x {source, w}
+  bool pred_local = false;       // with it: most in-arcs come from near vertices (path.hip)
   std::vector<int32_t> h_st2ed;     // host copy of st2ed (source lists of batched solves)
   std::vector<int32_t> h_graph_id;  // host copy of graph_id (part range checks)
   fap_bidx *bidx = nullptr;         // built on first batched part solve (bindex.hip)

@@ -271,7 +271,11 @@ __global__ __launch_bounds__(kPredThreads) void pred_kernel(
 }
 
 // Few cells (kPredFew): a thread each, the shortest chain (64 rows of 4,096
-// vertices: 27 us a call, 31 through pred_kernel; 2^20 cells: the same).
+// vertices: 27 us a call, 31 through pred_kernel; 2^20 cells: the same).  And
+// graphs without locality: all vertices of a few rows at a time, which the L2
+// then holds (1024 rows of 65,536 vertices at random, six arcs each: 1.89 ms;
+// pred_kernel's gathers walk many rows at once, 1.7 times that; arcs in
+// registers, up to 16 a vertex: 2.15).
 constexpr int64_t kPredFew = 1 << 20;
 
 __global__ __launch_bounds__(256) void pred_few_kernel(
@@ -376,6 +380,21 @@ static int ensure_in_csr(fap_ctx *ctx, fap_graph_dev *g, hipStream_t s) {
     (void)hipFree(d_in);
     return hip_fail(e, "transposed CSR copy", __FILE__, __LINE__);
   }
+  // is the graph laid out so that pred_kernel's blocks stage their rows?
+  int64_t staged = 0, blocks = 0;
+  for (int64_t j0 = 0; j0 < V; j0 += fapk::kPredBlock, blocks++) {
+    const int64_t j1 = std::min<int64_t>(j0 + fapk::kPredBlock, V);
+    int64_t lo = j0, hi = j1 - 1, most = 0;
+    for (int64_t j = j0; j < j1; j++) {
+      most = std::max<int64_t>(most, off[j + 1] - off[j]);
+      if (off[j + 1] > off[j]) {
+        lo = std::min<int64_t>(lo, in[off[j]].x);
+        hi = std::max<int64_t>(hi, in[off[j + 1] - 1].x);
+      }
+    }
+    staged += most <= fapk::kPredArcs && hi - lo < fapk::kPredSpan;
+  }
+  g->pred_local = 2 * staged >= blocks;
   g->in_offset = d_off;
   g->in_arcs = d_in;
   (void)ctx;
@@ -392,7 +411,7 @@ int run_pred_rows(fap_ctx *ctx, fap_graph_dev *g, const int32_t *d_dist, int64_t
   const int V = g->V;
   dim3 blk(256), grd((V + 255) / 256, std::min(nrows, 256));
   FAP_TRY(launch_fill_u32(cnt, 1, 0u, s));
-  if ((int64_t)nrows * V < fapk::kPredFew) {
+  if ((int64_t)nrows * V < fapk::kPredFew || !g->pred_local) {
     hipLaunchKernelGGL(fapk::pred_few_kernel, grd, blk, 0, s, d_dist, ld, d_own, nrows, V,
                        g->in_offset, g->in_arcs, d_pred, ldp, cnt);
   } else {

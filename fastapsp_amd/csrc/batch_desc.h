@@ -155,6 +155,18 @@ struct DenseJob {
 
 }  // namespace fapk
 
+namespace fapk {
+// One part of a batched solve, for the launches that serve all parts at once.
+struct PartJob {
+  int32_t *sub;  // part matrix, row stride ld_sub
+  int32_t *rows; // row block
+  int64_t ld_sub;
+  int32_t start, n, b;   // of st2ed; vertices, boundary vertices (first)
+  int32_t tile0, flags;  // first tile of its product, alignment flags
+  int32_t pad;
+};
+}  // namespace fapk
+
 namespace fapi {
 
 // Host side of a batched closure: jobs, the segments of every launch (launch

@@ -1024,11 +1024,14 @@ int bbf_buffers(fap_ctx *ctx, size_t bytes, size_t hbytes, char **h, char **d) {
 
 }  // namespace
 
+constexpr int kBatch = 16;  // boundary iterations between looks at the done word
+
 // Stage-1 rows for the boundary vertices of `count` parts (part indices
 // qidx, X rows from rowoff[p], nsrc rows in all; d_rowptr: device row
 // pointers of the output rows, V columns each, in the same order): the
 // block iterations, then the expansion, all enqueued on s.  The host looks
-// at the done word every kBatch iterations (one wait on s each time).
+// at the done word after 8 and then every kBatch iterations (one wait on s
+// each time).
 // Uses ctx->ws_bidx (nsrc x nbp int32) and ctx->ws_bbf / host_bbf.
 int bidx_rows(fap_ctx *ctx, const fap_graph_dev *g, int32_t count, const int32_t *qidx,
               const int32_t *rowoff, int32_t nsrc, int32_t *const *d_rowptr, hipStream_t s) {
@@ -1096,10 +1099,11 @@ int bidx_rows(fap_ctx *ctx, const fap_graph_dev *g, int32_t count, const int32_t
   // change is propagated eventually, so the result does not depend on the
   // band; values only decrease, so the iterations end.
   const int grid = (int)std::min<int64_t>(max_tiles, 8 * std::max(ctx->num_cus, 1));
-  constexpr int kBatch = 16;
-  for (int64_t it = 0;; it += kBatch) {
+  // a few parts settle within 8 iterations (8 parts of a 64 x 64 grid: 7)
+  int batch = 8;
+  for (int64_t it = 0;; it += batch, batch = kBatch) {
     if (it > ((int64_t)1 << 22)) return fail(FAP_E_STATE, "boundary iterations did not settle");
-    for (int i = 0; i < kBatch; i++) {
+    for (int i = 0; i < batch; i++) {
       hipLaunchKernelGGL(fapk::bidx_schedule_kernel, dim3(1), dim3(1024), 0, s, dctrl,
                          (int32_t *)(d + o_pend), (uint32_t *)(d + o_mask), (BidxTile *)(d + o_tile), (const int2 *)(d + o_prow), count, K, delta, tcol,
                          x->parts, x->outb_off, x->outb);

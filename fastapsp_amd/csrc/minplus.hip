@@ -4,6 +4,7 @@
 // fap/kernel/minplus.h:78-89; CPU semantics :51-65: every output starts at
 // INF and takes the strict minimum over k).  One 128 x 128 tile per
 // workgroup, additions on the matrix cores (mfma_tile.h).
+#include "batch_desc.h"
 #include "common.h"
 #include "mfma_tile.h"
 
@@ -34,6 +35,29 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4
   const int m0 = tm * MP_BM, n0 = tn * MP_BN;
   MxBig::run(A + (int64_t)m0 * lda, lda, B + n0, ldb, C + (int64_t)m0 * ldc + n0, ldc,
               imin(MP_BM, M - m0), imin(MP_BN, N - n0), K, accumulate != 0, flags, lds);
+}
+
+// The products of all parts of a batched solve (inner rows x boundary by
+// boundary x V) in one launch, for parts whose own would leave the chip idle:
+// 8 parts of a 64 x 64 grid, 128 tiles each, 150 -> 39 us.  Ragged last rows
+// take a whole tile (idle waves there are cheaper than launches).
+__global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void minplus_parts_kernel(
+    const PartJob *__restrict__ jobs, int count, int64_t ld_rows, int N, int tiles_n) {
+  __shared__ __attribute__((aligned(16))) int32_t lds[MxBig::LDS_WORDS];
+  int lo = 0, hi = count - 1;  // the last part whose first tile is not past this one
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (jobs[mid].tile0 <= (int)blockIdx.x) lo = mid;
+    else hi = mid - 1;
+  }
+  const PartJob j = jobs[lo];
+  const int M = j.n - j.b;
+  int tm, tn;
+  gemm_tile_coords(blockIdx.x - j.tile0, (M + MP_BM - 1) / MP_BM, tiles_n, &tm, &tn);
+  const int m0 = tm * MP_BM, n0 = tn * MP_BN;
+  MxBig::run(j.sub + (int64_t)(j.b + m0) * j.ld_sub, j.ld_sub, j.rows + n0, ld_rows,
+             j.rows + (int64_t)(j.b + m0) * ld_rows + n0, ld_rows, imin(MP_BM, M - m0),
+             imin(MP_BN, N - n0), j.b, false, j.flags, lds);
 }
 
 // The last rows of a product whose row count leaves at most 64 rows past
@@ -147,6 +171,15 @@ int launch_minplus(const int32_t *A, int64_t lda, const int32_t *B, int64_t ldb,
                        (int)tiles_n64);
     FAP_CHECK_LAUNCH();
   }
+  return FAP_OK;
+}
+
+int launch_minplus_parts(const fapk::PartJob *d_jobs, int32_t count, int32_t tiles,
+                         int64_t ld_rows, int32_t N, hipStream_t s) {
+  if (tiles <= 0) return FAP_OK;
+  hipLaunchKernelGGL(fapk::minplus_parts_kernel, dim3(tiles), dim3(fapk::MP_THREADS), 0, s, d_jobs,
+                     count, ld_rows, N, (N + fapk::MP_BN - 1) / fapk::MP_BN);
+  FAP_CHECK_LAUNCH();
   return FAP_OK;
 }
 

@@ -20,9 +20,10 @@ constexpr int GS_BX = 64, GS_BY = 4;
 // Rows < n_bdy: SSSP distances gathered through st2ed; other rows INF;
 // diagonal 0.  (The reference also writes the intra-part arcs of boundary
 // rows and then overwrites those rows with the SSSP distances, :36-65.)
-__global__ void gather_fill_kernel(const int32_t *__restrict__ st2ed, int start, int n_sub,
-                                   int n_bdy, const int32_t *__restrict__ rowblock,
-                                   int64_t ld_rb, int32_t *__restrict__ sub, int64_t ld_sub) {
+__device__ __forceinline__ void gather_fill(const int32_t *__restrict__ st2ed, int start,
+                                            int n_sub, int n_bdy,
+                                            const int32_t *__restrict__ rowblock, int64_t ld_rb,
+                                            int32_t *__restrict__ sub, int64_t ld_sub) {
   const int j = blockIdx.x * GS_BX + threadIdx.x;
   if (j >= n_sub) return;
   const int vj = st2ed[start + j];
@@ -39,15 +40,22 @@ __global__ void gather_fill_kernel(const int32_t *__restrict__ st2ed, int start,
   }
 }
 
+__global__ void gather_fill_kernel(const int32_t *__restrict__ st2ed, int start, int n_sub,
+                                   int n_bdy, const int32_t *__restrict__ rowblock,
+                                   int64_t ld_rb, int32_t *__restrict__ sub, int64_t ld_sub) {
+  gather_fill(st2ed, start, n_sub, n_bdy, rowblock, ld_rb, sub, ld_sub);
+}
+
 // Inner rows: the part's own arcs in CSR order, one thread per row so that
 // the last duplicate arc wins (:40-52); diagonal forced to 0 afterwards
 // (:67-72) so a self loop cannot override it.
-__global__ void gather_arcs_kernel(const int32_t *__restrict__ row_offset,
-                                   const int2 *__restrict__ edges,
-                                   const int32_t *__restrict__ graph_id,
-                                   const int32_t *__restrict__ st2ed,
-                                   const int32_t *__restrict__ ed2st, int start, int n_sub,
-                                   int n_bdy, int32_t *__restrict__ sub, int64_t ld_sub) {
+__device__ __forceinline__ void gather_arcs(const int32_t *__restrict__ row_offset,
+                                            const int2 *__restrict__ edges,
+                                            const int32_t *__restrict__ graph_id,
+                                            const int32_t *__restrict__ st2ed,
+                                            const int32_t *__restrict__ ed2st, int start,
+                                            int n_sub, int n_bdy, int32_t *__restrict__ sub,
+                                            int64_t ld_sub) {
   const int i = n_bdy + blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n_sub) return;
   const int u = st2ed[start + i];
@@ -62,14 +70,55 @@ __global__ void gather_arcs_kernel(const int32_t *__restrict__ row_offset,
   row[i] = 0;
 }
 
-__global__ void scatter_kernel(const int32_t *__restrict__ st2ed, int start, int rows, int n_sub,
-                               const int32_t *__restrict__ sub, int64_t ld_sub,
-                               int32_t *__restrict__ rowblock, int64_t ld_rb) {
+__global__ void gather_arcs_kernel(const int32_t *__restrict__ row_offset,
+                                   const int2 *__restrict__ edges,
+                                   const int32_t *__restrict__ graph_id,
+                                   const int32_t *__restrict__ st2ed,
+                                   const int32_t *__restrict__ ed2st, int start, int n_sub,
+                                   int n_bdy, int32_t *__restrict__ sub, int64_t ld_sub) {
+  gather_arcs(row_offset, edges, graph_id, st2ed, ed2st, start, n_sub, n_bdy, sub, ld_sub);
+}
+
+__device__ __forceinline__ void scatter(const int32_t *__restrict__ st2ed, int start, int rows,
+                                        int n_sub, const int32_t *__restrict__ sub,
+                                        int64_t ld_sub, int32_t *__restrict__ rowblock,
+                                        int64_t ld_rb) {
   const int j = blockIdx.x * GS_BX + threadIdx.x;
   if (j >= n_sub) return;
   const int vj = st2ed[start + j];
   for (int i = blockIdx.y * GS_BY + threadIdx.y; i < rows; i += gridDim.y * GS_BY)
     rowblock[(int64_t)i * ld_rb + vj] = sub[(int64_t)i * ld_sub + j];
+}
+
+__global__ void scatter_kernel(const int32_t *__restrict__ st2ed, int start, int rows, int n_sub,
+                               const int32_t *__restrict__ sub, int64_t ld_sub,
+                               int32_t *__restrict__ rowblock, int64_t ld_rb) {
+  scatter(st2ed, start, rows, n_sub, sub, ld_sub, rowblock, ld_rb);
+}
+
+// The same three for all parts of a batched solve (grid z): a part's own
+// launch is 4 to 9 us of a chip that it cannot fill, a few of them one after
+// another (8 parts of a 64 x 64 grid: 108 us, 25 together).
+__global__ void parts_fill_kernel(const int32_t *__restrict__ st2ed,
+                                  const PartJob *__restrict__ jobs, int64_t ld_rb) {
+  const PartJob p = jobs[blockIdx.z];
+  gather_fill(st2ed, p.start, p.n, p.b, p.rows, ld_rb, p.sub, p.ld_sub);
+}
+
+__global__ void parts_arcs_kernel(const int32_t *__restrict__ row_offset,
+                                  const int2 *__restrict__ edges,
+                                  const int32_t *__restrict__ graph_id,
+                                  const int32_t *__restrict__ st2ed,
+                                  const int32_t *__restrict__ ed2st,
+                                  const PartJob *__restrict__ jobs) {
+  const PartJob p = jobs[blockIdx.z];
+  gather_arcs(row_offset, edges, graph_id, st2ed, ed2st, p.start, p.n, p.b, p.sub, p.ld_sub);
+}
+
+__global__ void parts_scatter_kernel(const int32_t *__restrict__ st2ed,
+                                     const PartJob *__restrict__ jobs, int64_t ld_rb) {
+  const PartJob p = jobs[blockIdx.z];
+  scatter(st2ed, p.start, p.n, p.n, p.sub, p.ld_sub, p.rows, ld_rb);
 }
 
 }  // namespace fapk
@@ -88,6 +137,9 @@ int launch_fw(fap_ctx *ctx, int32_t *d, int32_t n, int64_t ld, hipStream_t s);
 int launch_minplus(const int32_t *A, int64_t lda, const int32_t *B, int64_t ldb, int32_t *C,
                    int64_t ldc, int32_t M, int32_t N, int32_t K, int accumulate,
                    hipStream_t s);
+int launch_minplus_parts(const fapk::PartJob *d_jobs, int32_t count, int32_t tiles,
+                         int64_t ld_rows, int32_t N, hipStream_t s);
+int vec_flags(const void *A, int64_t lda, const void *B, int64_t ldb, const void *C, int64_t ldc);
 
 static int check_part(const fap_graph_dev *g, int32_t start, int32_t n_sub, int32_t n_bdy) {
   if (!g->graph_id || !g->st2ed || !g->ed2st)
@@ -158,6 +210,10 @@ int run_subgraph_solve(fap_ctx *ctx, const fap_graph_dev *g, int32_t start, int3
   return FAP_OK;
 }
 
+// Products of fewer tiles than this on average share a launch: half of what
+// fits on the CUs at once.
+constexpr int64_t kSharedTiles = 512;
+
 // Enqueues the batched solve of `count` parts on stream s: every boundary
 // vertex's row (a row pointer per source into its part's row block) through
 // the boundary index when it holds every part -- the host waits on s while
@@ -202,7 +258,8 @@ int enqueue_subgraph_batch(fap_ctx *ctx, const fap_graph_dev *g, int32_t count,
   const size_t o_rp = up(4 * (size_t)nsrc);
   const size_t o_jobs = o_rp + up(sizeof(int32_t *) * (size_t)nsrc);
   const size_t o_segs = o_jobs + up(sizeof(fapk::BatchJob) * fd.jobs.size());
-  const size_t total = o_segs + std::max<size_t>(sizeof(fapk::BatchSeg) * fd.segs.size(), 16);
+  const size_t o_parts = o_segs + up(std::max<size_t>(sizeof(fapk::BatchSeg) * fd.segs.size(), 16));
+  const size_t total = o_parts + sizeof(fapk::PartJob) * (size_t)count;
   FAP_TRY(ensure_ws(ctx, ctx->ws_srcs, total));
   void *hs = nullptr;
   FAP_TRY(acquire_host_stage(ctx, total, &hs));
@@ -216,6 +273,25 @@ int enqueue_subgraph_batch(fap_ctx *ctx, const fap_graph_dev *g, int32_t count,
     }
   memcpy(h + o_jobs, fd.jobs.data(), sizeof(fapk::BatchJob) * fd.jobs.size());
   if (!fd.segs.empty()) memcpy(h + o_segs, fd.segs.data(), sizeof(fapk::BatchSeg) * fd.segs.size());
+  // part descriptors; products small enough on average to share a launch
+  fapk::PartJob *h_part = (fapk::PartJob *)(h + o_parts);
+  const int64_t tiles_n = (g->V + 127) / 128;
+  int64_t tiles = 0;
+  int32_t max_n = 0, max_inner = 0;
+  for (int32_t p = 0; p < count; p++) {
+    const int32_t inner = n_subs[p] - n_bdys[p];
+    h_part[p] = fapk::PartJob{subs[p], rowblocks[p], ld_sub[p], starts[p], n_subs[p], n_bdys[p],
+                              (int32_t)std::min<int64_t>(tiles, INT32_MAX),
+                              vec_flags(subs[p] + (int64_t)n_bdys[p] * ld_sub[p], ld_sub[p],
+                                        rowblocks[p], ld_rb,
+                                        rowblocks[p] + (int64_t)n_bdys[p] * ld_rb, ld_rb),
+                              0};
+    tiles += (inner + 127) / 128 * tiles_n;
+    max_n = std::max(max_n, n_subs[p]);
+    max_inner = std::max(max_inner, inner);
+  }
+  const bool together = count > 1 && count <= 65535;
+  const bool one_product = together && tiles < kSharedTiles * count && tiles <= INT32_MAX;
   char *d = (char *)ctx->ws_srcs.ptr;
   FAP_HIP(hipMemcpyAsync(d, h, total, hipMemcpyHostToDevice, s));
   FAP_TRY(release_host_stage(ctx, s));
@@ -227,18 +303,40 @@ int enqueue_subgraph_batch(fap_ctx *ctx, const fap_graph_dev *g, int32_t count,
     FAP_TRY(run_sssp_rows(ctx, g, (const int32_t *)d, (int32_t)nsrc, nullptr, 0,
                           (int32_t *const *)(d + o_rp), s));
   if (sssp_done) FAP_HIP(hipEventRecord(sssp_done, s));
-  for (int32_t p = 0; p < count; p++)
-    FAP_TRY(launch_gather(g, starts[p], n_subs[p], n_bdys[p], rowblocks[p], ld_rb, subs[p],
-                          ld_sub[p], s));
+  const fapk::PartJob *d_part = (const fapk::PartJob *)(d + o_parts);
+  const dim3 gs(fapk::GS_BX, fapk::GS_BY);
+  const dim3 all((max_n + fapk::GS_BX - 1) / fapk::GS_BX,
+                 std::min((max_n + fapk::GS_BY - 1) / fapk::GS_BY, 1024), (unsigned)count);
+  if (together && max_n > 0) {
+    hipLaunchKernelGGL(fapk::parts_fill_kernel, all, gs, 0, s, g->st2ed, d_part, ld_rb);
+    FAP_CHECK_LAUNCH();
+    if (max_inner > 0) {
+      hipLaunchKernelGGL(fapk::parts_arcs_kernel,
+                         dim3((max_inner + 255) / 256, 1, (unsigned)count), dim3(256), 0, s,
+                         g->row_offset, g->edges, g->graph_id, g->st2ed, g->ed2st, d_part);
+      FAP_CHECK_LAUNCH();
+    }
+  } else {
+    for (int32_t p = 0; p < count; p++)
+      FAP_TRY(launch_gather(g, starts[p], n_subs[p], n_bdys[p], rowblocks[p], ld_rb, subs[p],
+                            ld_sub[p], s));
+  }
   FAP_TRY(launch_fw_batch(ctx, fd, (const fapk::BatchJob *)(d + o_jobs),
                           (const fapk::BatchSeg *)(d + o_segs), s));
+  if (one_product) FAP_TRY(launch_minplus_parts(d_part, count, (int32_t)tiles, ld_rb, g->V, s));
   for (int32_t p = 0; p < count; p++) {
     const int32_t b = n_bdys[p];
-    FAP_TRY(launch_minplus(subs[p] + (int64_t)b * ld_sub[p], ld_sub[p], rowblocks[p], ld_rb,
-                           rowblocks[p] + (int64_t)b * ld_rb, ld_rb, n_subs[p] - b, g->V, b, 0,
-                           s));
-    FAP_TRY(launch_scatter(g, starts[p], n_subs[p], n_subs[p], subs[p], ld_sub[p], rowblocks[p],
-                           ld_rb, s));
+    if (!one_product)
+      FAP_TRY(launch_minplus(subs[p] + (int64_t)b * ld_sub[p], ld_sub[p], rowblocks[p], ld_rb,
+                             rowblocks[p] + (int64_t)b * ld_rb, ld_rb, n_subs[p] - b, g->V, b, 0,
+                             s));
+    if (!together)
+      FAP_TRY(launch_scatter(g, starts[p], n_subs[p], n_subs[p], subs[p], ld_sub[p], rowblocks[p],
+                             ld_rb, s));
+  }
+  if (together && max_n > 0) {
+    hipLaunchKernelGGL(fapk::parts_scatter_kernel, all, gs, 0, s, g->st2ed, d_part, ld_rb);
+    FAP_CHECK_LAUNCH();
   }
   return FAP_OK;
 }

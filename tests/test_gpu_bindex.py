@@ -125,3 +125,26 @@ def test_coarse_level(gpu_ctx, kind):
     dg.set_partition(gid, pc["st2ed"], pc["ed2st"])  # drops both
     assert dg.index_info() == (0, 0)
     dg.close()
+
+
+# Parts that share launches: without boundary, nothing but boundary, one vertex, more rows than a tile;
+# the products with fewer than 8 k, and with none.
+def test_uneven_parts_share_launches(gpu_ctx):
+    rng = np.random.default_rng(21)
+    sizes = [40, 12, 12, 1, 300, 150]
+    first = np.concatenate([[0], np.cumsum(sizes)])
+    arcs = []
+    for q, n in enumerate(sizes):
+        for i in range(1, n):
+            if q not in (1, 2):  # each vertex hangs on an earlier one of its part
+                arcs.append((first[q] + rng.integers(0, i), first[q] + i))
+    arcs += [(first[1] + i, first[2] + j) for i in range(12) for j in range(12) if (i + j) % 3 == 0]
+    arcs += [(first[4] + 7, first[5] + 3), (first[4] + 200, first[5] + 90), (first[2] + 4, first[4])]
+    u, v = np.array(arcs).T
+    V = int(first[-1])
+    from fastapsp_amd import synth
+    ro, col, w = synth.to_csr(V, u, v, rng.integers(1, 90, u.size), False)
+    gid = np.repeat(np.arange(len(sizes)), sizes).astype(np.int32) + 1
+    got, pc = solve_all(gpu_ctx, ro, col, w, gid, len(sizes))
+    for p in range(1, len(sizes) + 1):
+        np.testing.assert_array_equal(got[p - 1], O.run_part(p, ro, col, w, gid, pc))

@@ -28,14 +28,13 @@ Default run (what the one JSON line reports):
 
 roofline: the Floyd-Warshall closure (fw_diag/fw_panel/fw_rest kernels of
 one closure; the largest share of the step), timed with HIP events on its
-own stream; roofline_minplus the same for the product kernel.  Min-plus is
-not a multiply-accumulate, so the bound is the VALU, not MFMA.  peak = the
-measured ceiling of the kernels' instruction mix (one v_add_u32 per update,
-one v_min3_i32 per two), probed on the same device in the same run
-(fap_probe_minplus_ceiling); on gfx950 v_add_u32 issues at twice the rate of
-v_min3_i32, so that ceiling (~76 TOP/s) is above the spec figure of 1 int32
-op per lane per clock, 256 CUs x 64 lanes x 2.4 GHz = 39.3 T, which is
-reported beside it as spec_peak.
+own stream; roofline_minplus the same for the product kernel.  The additions
+of an update are outer sums on the matrix cores, the minima v_min3_i32 on the
+VALU; peak = that mix measured in registers and LDS alone (one 32x32x4 f16
+MFMA and 16 v_min3_i32 per 2048 updates, MX_MIX_TOPS).  valu_mix is the
+ceiling of the same work with its additions on the VALU, probed on the same
+device in the same run (fap_probe_minplus_ceiling); spec_peak is 1 int32 op
+per lane per clock, 256 CUs x 64 lanes x 2.4 GHz = 39.3 T.
 
 cpu_baseline: the reference's own CPU code (oracle/_ref, compiled from its
 headers; floyd_CPU_path and min_plus_path_CPU_advanced, single-threaded like
@@ -64,16 +63,13 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 VALU_PEAK_TOPS = 256 * 64 * 2.4e9 / 1e12  # spec: 1 int32 op per lane per clock, 39.32 T
+MX_MIX_TOPS = 102.0  # MFMA outer sums and v_min3_i32, 4 waves per SIMD
 # HBM bytes per launch of the n = 8192 min-plus product and per n = 8192
 # tile-128 FW closure, from two rocprofv3 counter runs (FETCH_SIZE x 2.0 +
 # WRITE_SIZE x 1.0, scales from a copy of known size): product 6.47e9 read
 # + 0.27e9 written; closure 34.07e9 read + 17.44e9 written.
 MINPLUS_8192_TRAFFIC = 6.74e9
 FW_8192_T128_TRAFFIC = 51.51e9
-# HBM bytes of the SSSP launch over the 512 x 512 grid's parts 1-32 (3,669
-# boundary vertices), from the same two counters: 283.4e9 read + 135.4e9
-# written.
-SSSP_GRID512_G32_TRAFFIC = 418.8e9
 HBM_PEAK_GBS = 8000.0
 
 
@@ -217,20 +213,21 @@ def dense_section(args, ctx, lib):
         "config": {"workload": f"dense FW closure + min-plus product, n={n}, arc p=0.01, "
                                f"w 1..1000 (value); batch_c4, serve_c5 and grid_c3 carry the "
                                f"batched/served-vs-plain forms", "n": n, "ops_per_step": ops_step},
-        "roofline": {"bound": "valu",
+        "roofline": {"bound": "valu and matrix cores",
                      "kernel": "Floyd-Warshall closure (fw_rest phase-3 tiles with the fused "
                                "next diagonal, fw_panel, fw_diag; one closure per step)",
-                     "achieved": round(ach_fw, 2), "peak": round(ceiling, 2), "unit": "TOP/s",
-                     "frac": round(ach_fw / ceiling, 3),
+                     "achieved": round(ach_fw, 2), "peak": MX_MIX_TOPS, "unit": "TOP/s",
+                     "frac": round(ach_fw / MX_MIX_TOPS, 3), "valu_mix": round(ceiling, 2),
                      "traffic": (FW_8192_T128_TRAFFIC if n == 8192 and tuned
                                  and tuned.get("params", [0])[0] == 128 else None),
-                     "peak_kind": "measured v_add_u32 + v_min3_i32 mix ceiling",
+                     "peak_kind": "measured 32x32x4 f16 MFMA + v_min3_i32 mix",
                      "spec_peak": round(VALU_PEAK_TOPS, 2),
                      "frac_of_spec_peak": round(ach_fw / VALU_PEAK_TOPS, 3),
                      "ms_per_launch": round(fw_avg, 3), "ops_per_launch": 2.0 * n ** 3},
-        "roofline_minplus": {"bound": "valu", "kernel": "minplus_gemm_kernel",
-                             "achieved": round(ach, 2), "peak": round(ceiling, 2),
-                             "unit": "TOP/s", "frac": round(ach / ceiling, 3),
+        "roofline_minplus": {"bound": "valu and matrix cores", "kernel": "minplus_gemm_kernel",
+                             "achieved": round(ach, 2), "peak": MX_MIX_TOPS,
+                             "unit": "TOP/s", "frac": round(ach / MX_MIX_TOPS, 3),
+                             "valu_mix": round(ceiling, 2),
                              "traffic": MINPLUS_8192_TRAFFIC if n == 8192 else None,
                              "spec_peak": round(VALU_PEAK_TOPS, 2),
                              "frac_of_spec_peak": round(ach / VALU_PEAK_TOPS, 3),
@@ -488,10 +485,6 @@ def grid_section(args, grid, modes=("plain", "pipelined")):
             "algorithmic_GB_per_s": round(sssp_bytes / (sssp_ms * 1e-3) / 1e9, 2),
             "frac_of_hbm_peak": round(sssp_bytes / (sssp_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 5),
             "tuned": tuned}
-    if args.grid == 512 and S == 3669:   # the counted launch: its measured HBM traffic
-        sssp["traffic"] = SSSP_GRID512_G32_TRAFFIC
-        sssp["traffic_GB_per_s"] = round(SSSP_GRID512_G32_TRAFFIC / (sssp_ms * 1e-3) / 1e9, 1)
-        sssp["traffic_frac_of_hbm_peak"] = round(sssp["traffic_GB_per_s"] / HBM_PEAK_GBS, 3)
     # the same sources' rows through the boundary index (stage 1 of the
     # batched forms), into the first parts' row blocks
     grp = parts[:G]
@@ -990,7 +983,7 @@ def batch_section(args, ctx, lib, ceiling):
             "plain_GOp_s": None if plain_ms is None else round(ops / (plain_ms * 1e-3) / 1e9, 1),
             "batched_GOp_s": round(ops / (bt * 1e-3) / 1e9, 1),
             "batched_over_plain": None if plain_ms is None else round(plain_ms / bt, 2),
-            "batched_frac_of_ceiling": round(ops / (bt * 1e-3) / 1e12 / ceiling, 3),
+            "batched_frac_of_ceiling": round(ops / (bt * 1e-3) / 1e12 / MX_MIX_TOPS, 3),
             "batched_frac_of_spec_peak": round(ops / (bt * 1e-3) / 1e12 / VALU_PEAK_TOPS, 3),
             "batched_launches": info["launches"], "batched_tasks": info["tasks"],
             "persistent_ms": None if pers_ms is None else round(pers_ms, 3),

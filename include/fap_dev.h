@@ -186,8 +186,8 @@ int fap_fw_batched_noalloc(fap_ctx *ctx, int32_t count, int32_t *const *d_mats, 
  * queue's XCD ran no workgroup).  Rows must be 128-byte aligned (each
  * matrix's address a multiple of 128 bytes, ld a multiple of 32), else
  * FAP_E_ARG: matrices on different XCDs then never share a cache line.
- * Slower than the plans' phase launches on the 512-graph batch (22.6 vs
- * 16.5 ms).  Synchronous. */
+ * Slower than the plans' phase launches on the 512-graph batch (23.8 vs
+ * 12.8 ms).  Synchronous. */
 int fap_fw_batched_persistent(fap_ctx *ctx, int32_t count, int32_t *const *d_mats,
                               const int32_t *n, const int64_t *ld, void *stream);
 
@@ -307,8 +307,8 @@ int fap_subgraph_pred(fap_ctx *ctx, fap_graph_dev *g, int32_t start, int32_t n_s
  * the part's own arcs), plus the graph of boundary vertices (cut arcs and
  * those in-part distances).  Batched part solves then compute stage 1 -- the
  * SSSP rows from every boundary vertex, fap/kernel/batch_sssp.h:254-277 --
- * as an SSSP on that much smaller graph (its distance array in LDS) followed
- * by one min-plus expansion per part, exactly the same rows.  Built on the
+ * on that much smaller graph, followed by one min-plus expansion per part,
+ * exactly the same rows.  Built on the
  * first batched solve (option "sssp_index"); this call builds it at once.
  * *built = 0 when the graph does not qualify (more than ~36 k boundary
  * vertices, duplicate arcs, a partition whose parts do not list their

@@ -26,9 +26,9 @@
 // sums.  Measured in registers and LDS alone (4 waves per SIMD): 102 TOP/s at
 // 2 ops per update against 70.3 of add, add, min3 (MFMA alone 149, v_min3
 // alone 137; the clock falls to 2.1 GHz with both units busy).  Kernels on the
-// 128 x 128 tile, integer tile before: the 8192^3 product 16.5 -> 11.15 ms
-// (98.6 TOP/s), 909 x 262144 x 115 0.888 -> 0.689 ms, the n = 8192 closure
-// 19.0 -> 15.1 ms.  Every product of more than 16 rows takes it: short k and
+// 128 x 128 tile, integer tile before: the 8192^3 product 16.5 -> 10.9 ms
+// (101 TOP/s), 909 x 262144 x 115 0.888 -> 0.687 ms, the n = 8192 closure
+// 19.0 -> 15.4 ms.  Every product of more than 16 rows takes it: short k and
 // edge tiles gain too, and values past the digits cost the first chunk.
 #ifndef FAP_MFMA_TILE_H_
 #define FAP_MFMA_TILE_H_
@@ -49,7 +49,6 @@ constexpr uint32_t MX_BAD = 0xBFC00000u;            // bits of v + 1 that leave 
 __device__ __forceinline__ uint32_t mx_digits(uint32_t w) {
   return __umul24((w >> 11) & 0x7FFu, 65536u - 2048u) + w;
 }
-
 
 // The same tile with integer additions, as a function of its own: inlined,
 // its registers and the matrix tile's accumulators would be live together

@@ -2,10 +2,12 @@
 //
 // One workgroup of 256 threads (4 waves) computes a 128 x 128 (or 64 x 64) tile
 //   C[i][j] = min(base, min_k A[i][k] + B[k][j]),  base = C[i][j] or INF.
-// Min-plus is not a multiply-accumulate, so it runs on the VALU, not MFMA:
-// every update is one v_add_u32, and two consecutive k are folded with one
-// v_min3_i32, i.e. 1.5 VALU instructions per update, issued as interleaved
-// (add, add, min3) triples so that adds of different waves can pair.
+// All on the VALU: every update is one v_add_u32, and two consecutive k are
+// folded with one v_min3_i32, i.e. 1.5 VALU instructions per update, issued as
+// interleaved (add, add, min3) triples so that adds of different waves can pair.
+// Most products take the tile of mfma_tile.h, whose additions are on the matrix
+// cores; this one serves tails, the batched panels and cross tiles (bound by
+// memory), and the values that the other cannot hold.
 //
 // Layout:
 //   * waves form a 2 x 2 grid of sub-tiles; a lane owns a TM x TN

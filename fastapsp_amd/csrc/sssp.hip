@@ -9,8 +9,8 @@
 // any exact method reproduces the reference's rows bit for bit.
 //
 // Method (near-far, Davidson et al. 2014, restated): each workgroup owns one
-// source at a time and keeps, in global memory, two "near" queues (current
-// and next round) and two "far" piles.  A round relaxes the out-arcs of every
+// source at a time and keeps two "near" queues (current and next round; in LDS
+// while they fit, in the packed form) and, in global memory, two "far" piles.  A round relaxes the out-arcs of every
 // near vertex u (strictly: dist[v] is lowered to dist[u] + w only when that is
 // smaller).  An improved v goes to the next near queue if its new distance is
 // below the threshold, otherwise to the far pile.  When the near queue
@@ -35,7 +35,6 @@
 #include "common.h"
 
 namespace fapk {
-
 
 __device__ __forceinline__ unsigned lane_prefix(unsigned long long mask) {
   return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),

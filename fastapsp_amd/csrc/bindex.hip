@@ -455,22 +455,24 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0x7F800000;
         load(0);
-        if (Tile::store_chunk(lds, st, ra, rb)) lds[Tile::FLAG] = 1;
+        Tile::store_chunk(lds, 0, st, ra, rb);
         __syncthreads();
-        int kbeg = 0, par = 0;
-        for (int k0 = MX_BK;; k0 += MX_BK) {  // as MxTile::product
-          const bool more = k0 < K;
+        int kbeg = 0, par = 0, k0 = MX_BK;
+        bad = 0;
+        while (k0 < K) {  // as MxTile::product
           const int kc = min(k0, K - MX_BK);
-          if (more) load(kc);
-          bad = __builtin_amdgcn_readfirstlane(lds[Tile::FLAG + par]);
+          load(kc);
+          bad = Tile::unfit(lds, par);
           if (bad) break;
-          Tile::compute(lds + par * Tile::BUF, kbeg, acc);
-          if (!more) break;
+          Tile::compute(lds + par * Tile::BUF, 0, acc);
           par ^= 1;
           kbeg = (k0 - kc) & ~1;
-          if (Tile::store_chunk(lds + par * Tile::BUF, st, ra, rb)) lds[Tile::FLAG + par] = 1;
+          Tile::store_chunk(lds, par, st, ra, rb);
           __syncthreads();
+          k0 += MX_BK;
         }
+        if (!bad) bad = Tile::unfit(lds, par);
+        if (!bad) Tile::compute(lds + par * Tile::BUF, kbeg, acc);
         if (!bad) {
           const int row0 = (wave >> 1) * (32 * NI) + (lane >> 5) * 4;
           const int col0 = (wave & 1) * (32 * NJ) + (lane & 31);
@@ -518,62 +520,6 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4
   }
 }
 
-// One expansion tile with integer additions (see bidx_expand_kernel).
-template <int TM, int TN>
-__device__ __attribute__((noinline)) void bidx_expand_int(mp_in_ptr A_, int64_t ldx, mp_in_ptr B_,
-                                                          int64_t ldv, int m_valid, int n_valid,
-                                                          int K, int32_t *const *rowptr,
-                                                          const int32_t *ids, mp_lds_ptr lds_) {
-  using Tile = MpTile<TM, TN>;
-  const int32_t *A = (const int32_t *)A_, *B = (const int32_t *)B_;
-  int32_t *As = (int32_t *)lds_, *Bs = As + Tile::BM * MP_AS_LD;
-  const int flags = MP_VEC_A | MP_VEC_B;  // hoff, ldx, lbv_off, ldv, j0 are multiples of 4
-  int acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; i++)
-#pragma unroll
-    for (int c = 0; c < TN; c++) acc[i][c] = kInf;
-  int ra[TM], rb[TN];
-  const int nch = (K + MP_BK - 1) / MP_BK;
-  if (nch > 0) {
-    Tile::load_chunk(A, ldx, B, ldv, m_valid, n_valid, K, 0, flags, ra, rb);
-    Tile::store_chunk(As, Bs, ra, rb);
-  }
-  __syncthreads();
-  for (int ch = 0; ch < nch; ch++) {
-    const bool more = ch + 1 < nch;
-    if (more) Tile::load_chunk(A, ldx, B, ldv, m_valid, n_valid, K, (ch + 1) * MP_BK, flags, ra, rb);
-    const int krem = K - ch * MP_BK;
-    Tile::compute(As, Bs, krem >= MP_BK ? MP_BK : (krem + 1) & ~1, acc);
-    __syncthreads();
-    if (more) {
-      Tile::store_chunk(As, Bs, ra, rb);
-      __syncthreads();
-    }
-  }
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const int row0 = (wave >> 1) * (8 * TM) + (lane >> 3);  // the tile's output layout
-  const int col0 = (wave & 1) * (8 * TN) + (lane & 7) * 4;
-#pragma unroll
-  for (int h = 0; h < TN / 4; h++) {
-    int cid[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      const int col = col0 + 32 * h + c;
-      cid[c] = col < n_valid ? ids[col] : -1;
-    }
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-      const int row = row0 + 8 * i;
-      if (row >= m_valid) continue;
-      int32_t *out = rowptr[row];
-#pragma unroll
-      for (int c = 0; c < 4; c++)
-        if (cid[c] >= 0) out[cid[c]] = acc[i][4 * h + c];
-    }
-  }
-}
-
 // Rows of the expansion: tile (16 TM sources, 16 TN columns of part q) =
 // min over c < b_q of X[s][hoff_q + c] + LBV_q[c][j], written to
 // rowptr[s][colid[start_q + j]].  A part without boundary vertices gives INF
@@ -604,30 +550,55 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4
     for (int j = 0; j < NJ; j++)
 #pragma unroll
       for (int r = 0; r < 16; r++) acc[i][j][r] = 0x7F800000;
-  if (!Tile::fits(ldx, P.ldv, n_valid, K) ||
-      Tile::product(A, ldx, B, P.ldv, m_valid, n_valid, K, lds, acc)) {
-    __syncthreads();
-    bidx_expand_int<TM, TN>((mp_in_ptr)A, ldx, (mp_in_ptr)B, P.ldv, m_valid, n_valid, K,
-                            rowptr + r0, ids, (mp_lds_ptr)lds);
-    return;
-  }
+  int done = 0, ha[TM], hb[TN];
+  if (Tile::fits(ldx, P.ldv, n_valid, K))
+    done = Tile::product(A, ldx, B, P.ldv, m_valid, n_valid, K, lds, acc, ha, hb);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row0 = (wave >> 1) * (32 * NI) + (lane >> 5) * 4;
-  const int col0 = (wave & 1) * (32 * NJ) + (lane & 31);
-  int cid[NJ];
+  if (done == K) {
+    const int row0 = (wave >> 1) * (32 * NI) + (lane >> 5) * 4;
+    const int col0 = (wave & 1) * (32 * NJ) + (lane & 31);
+    int cid[NJ];
 #pragma unroll
-  for (int j = 0; j < NJ; j++) cid[j] = ids[min(col0 + 32 * j, n_valid - 1)];
+    for (int j = 0; j < NJ; j++) cid[j] = ids[min(col0 + 32 * j, n_valid - 1)];
 #pragma unroll
-  for (int i = 0; i < NI; i++)
+    for (int i = 0; i < NI; i++)
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int row = row0 + 32 * i + Tile::acc_row(r);
-      if (row >= m_valid) continue;
+      for (int r = 0; r < 16; r++) {
+        const int row = row0 + 32 * i + Tile::acc_row(r);
+        if (row >= m_valid) continue;
+        int32_t *out = rowptr[r0 + row];
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+          if (col0 + 32 * j < n_valid) out[cid[j]] = Tile::value(acc[i][j][r]);
+      }
+  }
+  // values that the digits do not hold (see MxTile::run)
+  int64_t ldv = P.ldv;
+  int m = m_valid, n = n_valid, k = K;
+  mp_in_ptr a = (mp_in_ptr)A, b = (mp_in_ptr)B;
+  asm volatile("" : "+s"(a), "+s"(ldx), "+s"(b), "+s"(ldv), "+s"(m), "+s"(n), "+s"(k), "+s"(done));
+  if (done >= k) return;
+  int v[TM][TN];
+  // hoff, ldx, lbv_off, ldv, j0 are multiples of 4
+  Tile::finish((const int32_t *)a, ldx, (const int32_t *)b, ldv, m, n, k, MP_VEC_A | MP_VEC_B, lds,
+               done, false, ha, hb, acc, v);
+  const int row0 = (wave >> 1) * (8 * TM) + (lane >> 3);  // the integer tile's output layout
+  const int col0 = (wave & 1) * (8 * TN) + (lane & 7) * 4;
+#pragma unroll
+  for (int h = 0; h < TN / 4; h++) {
+    int cid[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) cid[c] = col0 + 32 * h + c < n ? ids[col0 + 32 * h + c] : -1;
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+      const int row = row0 + 8 * i;
+      if (row >= m) continue;
       int32_t *out = rowptr[r0 + row];
 #pragma unroll
-      for (int j = 0; j < NJ; j++)
-        if (col0 + 32 * j < n_valid) out[cid[j]] = Tile::value(acc[i][j][r]);
+      for (int c = 0; c < 4; c++)
+        if (cid[c] >= 0) out[cid[c]] = v[i][4 * h + c];
     }
+  }
 }
 
 // Index extraction for one part: from its closed local matrix (st2ed

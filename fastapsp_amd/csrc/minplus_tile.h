@@ -167,24 +167,27 @@ struct MpTile {
                                              int64_t ldb, int32_t *C, int64_t ldc, int m_valid,
                                              int n_valid, int K, bool accumulate, int flags,
                                              int32_t *lds) {
-    int32_t *As = lds;
-    int32_t *Bs = lds + BM * MP_AS_LD;
-    const int t = threadIdx.x;
-    const int wave = t >> 6, lane = t & 63;
-    const int lx = lane & 7, ly = lane >> 3;
-    const int row0 = (wave >> 1) * (8 * TM) + ly;    // rows row0 + 8r
-    const int col0 = (wave & 1) * (8 * TN) + lx * 4;  // cols col0 + 32h + c
-
     int acc[TM][TN];
 #pragma unroll
     for (int r = 0; r < TM; r++)
 #pragma unroll
       for (int c = 0; c < TN; c++) acc[r][c] = kInf;
-
     int ra[TM], rb[TN];
+    fold(A, lda, B, ldb, m_valid, n_valid, K, flags, lds, false, ra, rb, acc);
+    store(C, ldc, m_valid, n_valid, accumulate, flags, acc);
+  }
+
+  // acc = min(acc, A (x) B), operands as above.  `have`: ra and rb hold the
+  // first chunk already.
+  __device__ static __forceinline__ void fold(const int32_t *A, int64_t lda, const int32_t *B,
+                                              int64_t ldb, int m_valid, int n_valid, int K,
+                                              int flags, int32_t *lds, bool have,
+                                              int (&ra)[TM], int (&rb)[TN], int (&acc)[TM][TN]) {
+    int32_t *As = lds;
+    int32_t *Bs = lds + BM * MP_AS_LD;
     const int nchunks = (K + MP_BK - 1) / MP_BK;
     if (nchunks > 0) {
-      load_chunk(A, lda, B, ldb, m_valid, n_valid, K, 0, flags, ra, rb);
+      if (!have) load_chunk(A, lda, B, ldb, m_valid, n_valid, K, 0, flags, ra, rb);
       store_chunk(As, Bs, ra, rb);
     }
     __syncthreads();
@@ -202,8 +205,17 @@ struct MpTile {
         __syncthreads();
       }
     }
+  }
 
-    // epilogue.  Accumulating into a full tile, the C pieces of RG rows are
+  // C = acc, or min(C, acc).
+  __device__ static __forceinline__ void store(int32_t *C, int64_t ldc, int m_valid, int n_valid,
+                                               bool accumulate, int flags,
+                                               const int (&acc)[TM][TN]) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int lx = lane & 7, ly = lane >> 3;
+    const int row0 = (wave >> 1) * (8 * TM) + ly;    // rows row0 + 8r
+    const int col0 = (wave & 1) * (8 * TN) + lx * 4;  // cols col0 + 32h + c
+    // Accumulating into a full tile, the C pieces of RG rows are
     // all loaded before any of them is stored: stores to C may alias later
     // loads as far as the compiler knows (the row stride is a run-time
     // value), so loads interleaved with stores would each wait for the

@@ -26,15 +26,16 @@ __device__ __forceinline__ void gemm_tile_coords(int bid, int tiles_m, int tiles
   *tn = within / gsize;
 }
 
+template <class Tile>
 __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void minplus_gemm_kernel(
     const int32_t *A, int64_t lda, const int32_t *B, int64_t ldb, int32_t *C, int64_t ldc,
     int M, int N, int K, int accumulate, int flags, int tiles_m, int tiles_n) {
-  __shared__ __attribute__((aligned(16))) int32_t lds[MxBig::LDS_WORDS];
+  __shared__ __attribute__((aligned(16))) int32_t lds[Tile::LDS_WORDS];
   int tm, tn;
   gemm_tile_coords(blockIdx.x, tiles_m, tiles_n, &tm, &tn);
   const int m0 = tm * MP_BM, n0 = tn * MP_BN;
-  MxBig::run(A + (int64_t)m0 * lda, lda, B + n0, ldb, C + (int64_t)m0 * ldc + n0, ldc,
-              imin(MP_BM, M - m0), imin(MP_BN, N - n0), K, accumulate != 0, flags, lds);
+  Tile::run(A + (int64_t)m0 * lda, lda, B + n0, ldb, C + (int64_t)m0 * ldc + n0, ldc,
+            imin(MP_BM, M - m0), imin(MP_BN, N - n0), K, accumulate != 0, flags, lds);
 }
 
 // The products of all parts of a batched solve (inner rows x boundary by
@@ -152,9 +153,14 @@ int launch_minplus(const int32_t *A, int64_t lda, const int32_t *B, int64_t ldb,
   const int64_t tiles_n = (N + fapk::MP_BN - 1) / fapk::MP_BN;
   if (tiles_m * tiles_n > INT32_MAX) return fail(FAP_E_ARG, "min-plus: too many tiles");
   const int flags = vec_flags(A, lda, B, ldb, C, ldc);
-  hipLaunchKernelGGL(fapk::minplus_gemm_kernel, dim3((unsigned)(tiles_m * tiles_n)),
-                     dim3(fapk::MP_THREADS), 0, s, A, lda, B, ldb, C, ldc, (int)Mb, (int)N,
-                     (int)K, accumulate, flags, (int)tiles_m, (int)tiles_n);
+  // Below 16 k the integer tile: such a product is its stores, and the matrix
+  // cores only add their first look (4096 x 16384 x 5 58 us, 63 through it;
+  // 4096 x 65536 x 12 235 us, 233 there, 264 on values past the digits).
+  auto kernel = K < fapk::MP_BK ? fapk::minplus_gemm_kernel<fapk::MpBig>
+                                : fapk::minplus_gemm_kernel<fapk::MxBig>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(fapk::MP_THREADS), 0, s, A,
+                     lda, B, ldb, C, ldc, (int)Mb, (int)N, (int)K, accumulate, flags, (int)tiles_m,
+                     (int)tiles_n);
   FAP_CHECK_LAUNCH();
   if (tail > 0 && tail <= fapk::ROWS16) {
     hipLaunchKernelGGL(fapk::minplus_rows16_kernel, dim3((unsigned)cols256), dim3(256), 0, s,

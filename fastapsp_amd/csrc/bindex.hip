@@ -323,60 +323,78 @@ __device__ __forceinline__ void bidx_enter(const int32_t *xa, const int2 (&f)[N]
   }
 }
 
-// The tile's product with integer additions, the collected positions and all
-// (16 k a chunk), in the accumulator layout of MpTile; for lists shorter than
-// a matrix-core chunk and values that its digits do not hold.
+// The tile's update with integer additions (16 k a chunk, in the layout of
+// MpTile), for lists shorter than 16 and values that the digits do not hold.
+// `have`: ra and rb hold the first chunk already.
 template <int TM, int TN>
-__device__ __attribute__((noinline)) int bidx_tile_int(mp_out_ptr Xt_, int64_t ldx, mp_in_ptr B_,
-                                                       int ldb, const int2 *in_arc, int K,
-                                                       int m_valid, int n_valid, int c_off,
-                                                       mp_lds_ptr lds_, mp_lds_ptr klist_,
-                                                       mp_lds_ptr kinf_) {
+__device__ __forceinline__ int bidx_tile_int(int32_t *Xt, int64_t ldx, const int32_t *B, int ldb,
+                                             const int2 *in_arc, int K, int m_valid, int n_valid,
+                                             int c_off, int32_t *lds, const int32_t *klist,
+                                             const int2 *kinf, bool have, int (&ra)[TM],
+                                             int (&rb)[TN]) {
   using Tile = MpTile<TM, TN>;
-  int32_t *Xt = (int32_t *)Xt_;
-  const int32_t *B = (const int32_t *)B_;
-  int32_t *As = (int32_t *)lds_, *Bs = As + Tile::BM * MP_AS_LD;
-  const int32_t *klist = (const int32_t *)klist_;
-  const int2 *kinf = (const int2 *)(int32_t *)kinf_;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  int32_t *As = lds, *Bs = As + Tile::BM * MP_AS_LD;
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));  // nothing that follows from it is kept across tiles
+  const int wave = t >> 6, lane = t & 63;
   const int arow = t / Tile::A_TPR, akq = (t % Tile::A_TPR) * TM;  // A staging (the tile's layout)
-  const int row0 = (wave >> 1) * (8 * TM) + (lane >> 3);  // the tile's output layout
-  const int col0 = (wave & 1) * (8 * TN) + (lane & 7) * 4;
   const int32_t *xa = Xt + (int64_t)min(arow, m_valid - 1) * ldx;
+  const int col = (t & 15) * TN;
+  auto load = [&](int k0) {  // k past K repeat the last one
+    int2 f[TM];
+#pragma unroll
+    for (int j = 0; j < TM; j++) f[j] = kinf[min(k0 + akq + j, K - 1)];
+    const int32_t *pb = B + (int64_t)klist[min(k0 + (t >> 4), K - 1)] * ldb;
+    if (col + TN <= n_valid) {
+#pragma unroll
+      for (int q = 0; q < TN; q += 4) {
+        const int4 v = *reinterpret_cast<const int4 *>(pb + col + q);
+        rb[q] = v.x; rb[q + 1] = v.y; rb[q + 2] = v.z; rb[q + 3] = v.w;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < TN; j++) rb[j] = pb[min(col + j, n_valid - 1)];
+    }
+    bidx_enter<TM>(xa, f, in_arc, ra);
+  };
   int acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; i++)
 #pragma unroll
     for (int c = 0; c < TN; c++) acc[i][c] = kInf;
+  if (!have) load(0);
+  Tile::store_chunk(As, Bs, ra, rb);
+  __syncthreads();
   for (int k0 = 0; k0 < K; k0 += MP_BK) {
-    int ra[TM], rb[TN];
-    int2 f[TM];
-#pragma unroll
-    for (int j = 0; j < TM; j++) f[j] = kinf[min(k0 + akq + j, K - 1)];
-    bidx_enter<TM>(xa, f, in_arc, ra);
-    const int kr = k0 + (t >> 4), col = (t & 15) * TN;
-    const int32_t *pb = B + (int64_t)klist[min(kr, K - 1)] * ldb;
-#pragma unroll
-    for (int j = 0; j < TN; j++) rb[j] = pb[min(col + j, n_valid - 1)];
-    __syncthreads();  // the previous chunk's readers are done
-    Tile::store_chunk(As, Bs, ra, rb);
+    const bool more = k0 + MP_BK < K;
+    if (more) load(k0 + MP_BK);
+    Tile::compute(As, Bs, more ? MP_BK : (K - k0 + 1) & ~1, acc);
     __syncthreads();
-    Tile::compute(As, Bs, MP_BK, acc);  // k past K repeat the last one
+    if (more) {
+      Tile::store_chunk(As, Bs, ra, rb);
+      __syncthreads();
+    }
+  }
+  const int row0 = (wave >> 1) * (8 * TM) + (lane >> 3);  // the tile's output layout
+  const int col0 = (wave & 1) * (8 * TN) + (lane & 7) * 4;
+  int o[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++) {
+    const int32_t *cr = Xt + (int64_t)min(row0 + 8 * i, m_valid - 1) * ldx + c_off;
+#pragma unroll
+    for (int c = 0; c < TN; c++) o[i][c] = cr[min(col0 + 32 * (c >> 2) + (c & 3), n_valid - 1)];
   }
   int lowest = kInf;
 #pragma unroll
-  for (int i = 0; i < TM; i++) {
-    const int row = row0 + 8 * i;
-    int32_t *cr = Xt + (int64_t)row * ldx + c_off;
+  for (int i = 0; i < TM; i++)
 #pragma unroll
     for (int c = 0; c < TN; c++) {
-      const int col = col0 + 32 * (c >> 2) + (c & 3);
-      if (row < m_valid && col < n_valid && acc[i][c] < cr[col]) {
-        cr[col] = acc[i][c];
+      const int row = row0 + 8 * i, x = col0 + 32 * (c >> 2) + (c & 3);
+      if (row < m_valid && x < n_valid && acc[i][c] < o[i][c]) {
+        Xt[(int64_t)row * ldx + c_off + x] = acc[i][c];
         lowest = min(lowest, acc[i][c]);
       }
     }
-  }
   return lowest;
 }
 
@@ -393,12 +411,14 @@ __device__ __attribute__((noinline)) int bidx_tile_int(mp_out_ptr Xt_, int64_t l
 // either value is the length of a walk, and a lowered one is pending again,
 // so the iteration only converges on exact distances.
 // K is ~47: the tile is a chain of loads (its list, the gathers, C) around a
-// short product.  The product runs on the matrix cores (mfma_tile.h); the
-// gathers of a chunk and C's cells are each loaded together (a branch or a
-// conditional store between them made each wait for the one before).
-// 64 x 64 grid in 8 parts: 13.6 -> 10 us a launch; 512 x 512 grid, 32 parts (1,681
-// tiles a launch on average): 89 us before and after, the X rows' traffic
-// (~100 KB a tile).
+// short product.  The product runs on the matrix cores (mfma_tile.h), 64
+// columns starting with 16 k at once; values past its digits start again with
+// integer additions (K is short), in 64 columns from what was gathered.  The
+// gathers of a chunk and C's cells are each loaded together, in both forms (a
+// branch or a conditional store between them made each wait for the one
+// before).  Integer tile alone -> both: all of a 64 x 64 grid in 8 parts 1.52 ->
+// 1.06 ms, weights to 300,000 1.53 -> 1.15; one of 30 parts of a 40,000-vertex
+// random geometric graph 2.63 -> 2.18 and 2.64 -> 2.37.
 template <int TM, int TN>
 __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void bidx_block_kernel(
     const int32_t *__restrict__ ctrl, const BidxTile *__restrict__ tiles, int32_t *X, int64_t ldx,
@@ -433,8 +453,8 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4
       const int K = more_list ? kListSeg : ktot;
       Tile::init_lds(lds);
       __syncthreads();  // the list is there, the flags are cleared
-      int bad = 1;
-      if (K >= MX_BK && n_valid >= EB) {
+      int bad = 1, have = 0, ha[TM], hb[TN];
+      if (K >= MP_BK && n_valid >= 4) {
         const typename Tile::Stage st(0, Q.ldb, m_valid, n_valid);
         const int32_t *xa = Xt + (int64_t)min(t / Tile::A_TPR, m_valid - 1) * ldx;
         int ra[EA], rb[EB];
@@ -454,12 +474,29 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4
           for (int j = 0; j < NJ; j++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0x7F800000;
-        load(0);
-        Tile::store_chunk(lds, 0, st, ra, rb);
-        __syncthreads();
         int kbeg = 0, par = 0, k0 = MX_BK;
-        bad = 0;
-        while (k0 < K) {  // as MxTile::product
+        if constexpr (Tile::PAIR) {  // two chunks at once, as MxTile::product
+          int2 f[TM];
+#pragma unroll
+          for (int j = 0; j < TM; j++) f[j] = kinf[(t & 3) * 4 + j];
+          Tile::template load_vec<4>(B + (int64_t)klist[t >> 4] * Q.ldb,
+                                     4u * (uint32_t)Tile::pair_col(n_valid), hb);
+          bidx_enter<TM>(xa, f, in_arc, ha);
+          Tile::store_pair(lds, n_valid, ha, hb);
+          __syncthreads();
+          bad = Tile::unfit(lds, 0);
+          have = bad && n_valid == TC;
+          if (!bad) Tile::compute(lds, 0, acc);
+          __syncthreads();
+          par = 1;
+          k0 = 2 * MX_BK;
+        } else {
+          load(0);
+          Tile::store_chunk(lds, 0, st, ra, rb);
+          __syncthreads();
+          bad = 0;
+        }
+        while (k0 < K && !bad) {
           const int kc = min(k0, K - MX_BK);
           load(kc);
           bad = Tile::unfit(lds, par);
@@ -472,14 +509,15 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4
           k0 += MX_BK;
         }
         if (!bad) bad = Tile::unfit(lds, par);
-        if (!bad) Tile::compute(lds + par * Tile::BUF, kbeg, acc);
         if (!bad) {
-          const int row0 = (wave >> 1) * (32 * NI) + (lane >> 5) * 4;
-          const int col0 = (wave & 1) * (32 * NJ) + (lane & 31);
-          // byte offsets in C (64 rows of at most 2^18 words); the stride is made
-          // opaque here, or the offsets of all rows are kept across tiles
+          Tile::compute(lds + par * Tile::BUF, kbeg, acc);
+          // byte offsets in C (64 rows of at most 2^18 words); the stride and the
+          // first row are made opaque here, or what follows from them is kept
+          // (in scratch memory) across tiles
           uint32_t stride = (uint32_t)ldx * 4u;
-          asm volatile("" : "+s"(stride));
+          int row0 = (wave >> 1) * (32 * NI) + (lane >> 5) * 4;
+          asm volatile("" : "+s"(stride), "+v"(row0));
+          const int col0 = (wave & 1) * (32 * NJ) + (lane & 31);
           char *cb = reinterpret_cast<char *>(Xt + Q.hoff + c0);
 #pragma unroll
           for (int i = 0; i < NI; i++)
@@ -505,12 +543,18 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4
             }
         }
       }
-      if (bad && K > 0) {
+      // (see MxTile::run)
+      mp_out_ptr xp = (mp_out_ptr)Xt;
+      mp_in_ptr bp = (mp_in_ptr)B;
+      int64_t lx = ldx;
+      int lb = Q.ldb, k = K, m = m_valid, n = n_valid, c = Q.hoff + c0;
+      asm volatile("" : "+s"(xp), "+s"(lx), "+s"(bp), "+s"(lb), "+s"(k), "+s"(m), "+s"(n));
+      asm volatile("" : "+s"(c), "+s"(bad));
+      if (bad && k > 0) {
         __syncthreads();  // the staging is rewritten
-        lowest = min(lowest, bidx_tile_int<TM, TN>(
-                                 (mp_out_ptr)Xt, ldx, (mp_in_ptr)B, Q.ldb, in_arc, K, m_valid, n_valid,
-                                 Q.hoff + c0, (mp_lds_ptr)lds, (mp_lds_ptr)klist,
-                                 (mp_lds_ptr)(int32_t *)kinf));
+        lowest = min(lowest, bidx_tile_int<TM, TN>((int32_t *)xp, lx, (const int32_t *)bp, lb,
+                                                   in_arc, k, m, n, c, lds, klist, kinf,
+                                                   have != 0, ha, hb));
       }
       __syncthreads();  // the list and the staging are rewritten by what follows
     }
@@ -1020,7 +1064,10 @@ int bidx_rows(fap_ctx *ctx, const fap_graph_dev *g, int32_t count, const int32_t
   // workspace: control | block rows {first X row, rows} | source rows {part,
   // H position} | pending | marks | tiles
   // block-update tile: 64 rows x tcol columns (tcol = 64 or 128)
-  const int tcol = ctx->opt_bidx_tile == 64 ? 64 : 128;
+  // few sources make few tiles: 64 columns then (one of 16 parts of a 128 x 128
+  // grid 1.82 ms, 2.00 with 128; all 16, 1,100 sources, 4.09 and 4.08; 31 parts of
+  // a 320 x 320 grid 97.1 and 92.7)
+  const int tcol = ctx->opt_bidx_tile ? ctx->opt_bidx_tile : nsrc >= 1024 ? 128 : 64;
   int64_t rt_sum = 0, ct_sum = 0;
   for (int32_t p = 0; p < count; p++) rt_sum += (x->h_parts[qidx[p]].b + 63) / 64;
   for (int32_t q = 0; q < K; q++) ct_sum += (x->h_parts[q].b + tcol - 1) / tcol;

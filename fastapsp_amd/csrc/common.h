@@ -117,7 +117,7 @@ struct fap_ctx {
   int opt_sssp_wgs = 0;          // SSSP workgroups per CU: 1..8; 0 = 1024 threads per CU
   int opt_sssp_arcs = 2;         // accepted (1, 2, 4); the SSSP kernel takes four at once
   int opt_sssp_index = 1;        // batched part solves: stage 1 through the boundary index (1) or SSSP (0)
-  int opt_bidx_tile = 0;         // boundary iterations' tile columns: 64 or 128; 0 = 128
+  int opt_bidx_tile = 0;         // boundary iterations' tile columns: 64 or 128; 0 = by the number of sources
   int opt_bidx_delta = 0;        // distance band of the boundary iterations; 0 = mean arc weight x sqrt(V / K)
   int64_t opt_batch_wait_us = 0;  // single-launch batched closure: longest wait of a task; 0 = 2 s
   fap_tune_cache *tune = nullptr;  // not owned

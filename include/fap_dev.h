@@ -91,7 +91,8 @@ int fap_ctx_stream(fap_ctx *ctx, void **stream);
  *                           for its matrix's earlier phases, in microseconds [2 s]
  *   "sssp_index"   0/1      batched part solves compute stage 1 through the graph's
  *                           boundary index (built by the first such call) [1]
- *   "bidx_tile"    0/64/128 columns of the boundary index's 64-row block-update tiles [128]
+ *   "bidx_tile"    0/64/128 columns of the boundary index's 64-row block-update tiles
+ *                           [128 from 1,024 sources, 64 below]
  *   "bidx_delta"   >= 0     distance band of the boundary index's block iterations; any
  *                           value gives the same rows [mean arc weight x sqrt(V / K),
  *                           times 32 / parts for calls of fewer than 32 parts] */

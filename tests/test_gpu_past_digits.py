@@ -77,3 +77,36 @@ def test_closure_in_64_blocks(gpu_ctx, n, pad, lookahead, hi, late):
     np.testing.assert_array_equal(got[:, :n], O.floyd(m))
     assert (got[:, n:] == -9).all()
     d.free()
+
+
+# Boundary block updates (fewer than 32 parts: no coarse level): every block past the digits, or some of
+# its border positions only; lists below and above 16 positions, several chunks
+@pytest.mark.parametrize("side,K", [(24, 5), (48, 6)])
+@pytest.mark.parametrize("share", [1.0, 0.03])
+@pytest.mark.parametrize("tile", [0, 64, 128])
+def test_boundary_blocks(gpu_ctx, side, K, share, tile):
+    from fastapsp_amd import synth
+    V = side * side
+    u, v, w = synth.grid_graph(side, side, 0.05, 0.02, 1, 100, side + K)
+    rng = np.random.default_rng(side)
+    w = np.where(rng.random(len(w)) < share, rng.integers(1 << 20, 1 << 23, len(w)), w).astype(np.int32)
+    ro, col, w = synth.to_csr(V, u, v, w, False)
+    gid = (np.arange(V) * K // V + 1).astype(np.int32)
+    pc = O.precondition(K, gid, ro, col)
+    dg = gpu_ctx.upload_graph(ro, col, w)
+    dg.set_partition(gid, pc["st2ed"], pc["ed2st"])
+    assert dg.build_index()
+    gpu_ctx.set_option("bidx_tile", tile)
+    try:
+        for ids in ([2], list(range(1, K + 1))):
+            outs = [gpu_ctx.alloc((int(pc["ver_num"][p]), V)) for p in ids]
+            dg.subgraph_solve_batch([int(pc["ver_off"][p]) for p in ids],
+                                    [int(pc["ver_num"][p]) for p in ids],
+                                    [int(pc["bdy_num"][p]) for p in ids], [o.ptr for o in outs], V)
+            for p, o in zip(ids, outs):
+                if p <= 2:
+                    np.testing.assert_array_equal(o.get(), O.run_part(p, ro, col, w, gid, pc))
+                o.free()
+    finally:
+        gpu_ctx.set_option("bidx_tile", 0)
+    dg.close()

@@ -50,7 +50,8 @@ def elf_kernels(elf):
 # closes the next diagonal block, in a function of its own)
 @pytest.mark.parametrize("kernel", ["minplus_gemm_kernel", "minplus_parts_kernel", "hidx_cross_kernel",
                                     "fw_pair128_kernel", "fw_rest_kernelILi8ELb0E",
-                                    "fw_rest_kernelILi4E", "fw_panel_kernel", "bidx_expand_kernel"])
+                                    "fw_rest_kernelILi4E", "fw_panel_kernel", "bidx_expand_kernel",
+                                    "bidx_block_kernelILi4ELi4E"])
 def test_tiles_stay_in_registers(kernel):
     found = {n: k[".private_segment_fixed_size"] for n, k in kernel_metadata().items() if kernel in n}
     assert found

@@ -15,12 +15,21 @@
 namespace fapk {
 
 // A wave builds a row, 1,024 columns at a time in its own LDS buffer: INF,
-// the row's arcs one after another (the last duplicate wins; a wave's LDS
-// writes land in order), the diagonal, then out with 16-byte stores.  Bound:
+// the row's arcs one after another (the last duplicate wins), the diagonal,
+// then out with 16-byte stores, each step behind wave_order.  Bound:
 // writing the matrices once.  512 graphs (1.19 GB): 0.31 ms; 1.62 ms as a
 // fill kernel that searched its job and divided once per cell, followed by a
 // kernel with a thread per row of arcs.
 constexpr int DR_COLS = 1024, DR_WAVES = 4;
+
+// What lanes of a wave have written to LDS comes before what any of them
+// writes or reads after this.  (No instruction: a wave's LDS accesses are in
+// order; it keeps the compiler to theirs.)
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 __global__ __launch_bounds__(64 * DR_WAVES) void dense_rows_kernel(const DenseJob *__restrict__ jobs,
                                                                    int count, int32_t rows) {
@@ -46,15 +55,18 @@ __global__ __launch_bounds__(64 * DR_WAVES) void dense_rows_kernel(const DenseJo
       for (int i = 0; i < DR_COLS; i += 256)
         *reinterpret_cast<int4 *>(w + i + 4 * lane) =
             make_int4(0x3FFFFFFF, 0x3FFFFFFF, 0x3FFFFFFF, 0x3FFFFFFF);
+      wave_order();
       for (int e = e0; e < e1; e += 64) {
         const int2 ed = e + lane < e1 ? edges[e + lane] : make_int2(-1, 0);
         const unsigned at = (unsigned)(ed.x - c0);
         const int m = e1 - e < 64 ? e1 - e : 64;
-        for (int k = 0; k < m; k++)
+        for (int k = 0; k < m; k++) {  // one after another: duplicates
           if (lane == k && at < (unsigned)DR_COLS) w[at] = ed.y;
+          wave_order();
+        }
       }
       if (lane == 0 && (unsigned)(u - c0) < (unsigned)DR_COLS) w[u - c0] = 0;
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      wave_order();
       const int m = n - c0 < DR_COLS ? n - c0 : DR_COLS;
 #pragma unroll
       for (int i = 0; i < DR_COLS; i += 256) {
@@ -68,7 +80,7 @@ __global__ __launch_bounds__(64 * DR_WAVES) void dense_rows_kernel(const DenseJo
             if (j + q < m) row[c0 + j + q] = v[q];
         }
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      wave_order();
     }
   }
 }

@@ -69,6 +69,7 @@ struct fap_graph_dev {
   bool pred_local = false;       // with it: most in-arcs come from near vertices (path.hip)
   std::vector<int32_t> h_st2ed;     // host copy of st2ed (source lists of batched solves)
   std::vector<int32_t> h_graph_id;  // host copy of graph_id (part range checks)
+  bool part_local = false;          // with them: a part's vertices are mostly near in number (submat.hip)
   fap_bidx *bidx = nullptr;         // built on first batched part solve (bindex.hip)
   int bidx_state = 0;               // 0 not tried, 1 built, -1 not applicable
   std::atomic<fap_hidx *> hidx{nullptr};  // with bidx, where the graph has enough parts

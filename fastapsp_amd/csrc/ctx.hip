@@ -512,6 +512,9 @@ int fap_graph_set_partition(fap_ctx *ctx, fap_graph_dev *g, const int32_t *graph
   FAP_HIP(hipStreamSynchronize(ctx->stream));
   g->h_st2ed.assign(st2ed, st2ed + V);
   g->h_graph_id.assign(graph_id, graph_id + V);
+  int64_t near = 0;  // neighbours in a part's list on one 128-byte line of a row
+  for (int32_t i = 1; i < V; i++) near += (st2ed[i] >> 5) == (st2ed[i - 1] >> 5);
+  g->part_local = 2 * near >= V;
   hidx_release(g);
   bidx_release(g);  // an index belongs to the partition it was built for
   return FAP_OK;

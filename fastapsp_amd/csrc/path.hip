@@ -94,9 +94,19 @@ __device__ __forceinline__ unsigned int pred_scan(const PredRows &x, int i, int 
   } else if (dj >= 0x3FFFFFFF) {
     p = -1;
   } else {
-    for (int e = 0; e < deg && p == kUnresolved; e++) {
-      const int2 a = arcs[e];
-      if (a.y > 0 && d[a.x] + a.y == dj) p = a.x;
+    // four arcs at a time: a load does not wait to see whether the arc before
+    // was tight (300 rows of 65,536 vertices, 12 random in-arcs: 743 us, 1,226
+    // one by one; 20 in-arcs nearby: 504, 1,445, and 1,321 with all of them read)
+    for (int e = 0; e < deg && p == kUnresolved; e += 4) {
+      int2 a[4];
+      int du[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) a[k] = arcs[min(e + k, deg - 1)];
+#pragma unroll
+      for (int k = 0; k < 4; k++) du[k] = d[a[k].x];
+#pragma unroll
+      for (int k = 3; k >= 0; k--)  // the first tight one is the smallest
+        if (a[k].y > 0 && du[k] + a[k].y == dj) p = a[k].x;
     }
   }
   x.pred[(int64_t)i * x.ldp + j] = p;
@@ -271,11 +281,11 @@ __global__ __launch_bounds__(kPredThreads) void pred_kernel(
 }
 
 // Few cells (kPredFew): a thread each, the shortest chain (64 rows of 4,096
-// vertices: 27 us a call, 31 through pred_kernel; 2^20 cells: the same).  And
-// graphs without locality: all vertices of a few rows at a time, which the L2
-// then holds (1024 rows of 65,536 vertices at random, six arcs each: 1.89 ms;
-// pred_kernel's gathers walk many rows at once, 1.7 times that; arcs in
-// registers, up to 16 a vertex: 2.15).
+// vertices 27 us a call, 31 through pred_kernel; 2^20 cells the same, 2^21 37
+// and 35).  And graphs without locality: all vertices of a few rows at a time,
+// which the L2 then holds (1024 rows of 65,536 vertices at random, six arcs
+// each, one after another: 1.89 ms; pred_kernel's gathers walk many rows at
+// once, 1.7 times that; arcs in registers, up to 16 a vertex: 2.15).
 constexpr int64_t kPredFew = 1 << 20;
 
 __global__ __launch_bounds__(256) void pred_few_kernel(

@@ -140,8 +140,14 @@ __device__ __forceinline__ void bin_queue(const uint32_t *__restrict__ q, uint32
 // dependent memory trips; larger ones, the vector cache's address rate, about
 // a lane a cycle and CU for gathers (a load more or less per entry in every
 // step: 100 cycles a wave).  So
-//  - the near queues are in LDS, and an entry brings its vertex's arc range;
-//    entries past the queue's room, and only they, go through memory;
+//  - the near queues are in LDS, and an entry brings its vertex's arc range.
+//    A queue that outgrows its room (2 NT entries) goes through memory as a
+//    whole and is reordered there by vertex block, and the round that works on
+//    it, which will hardly make a smaller one, fills memory at once: a graph
+//    without locality has fronts of thousands, whose ranges, arcs and words
+//    are a line each in any other order (65,536 vertices, 6 random arcs each
+//    way, 300 sources: 21.3 ms, 26.8 with the first 2 NT entries in LDS and
+//    the rest in memory, neither reordered);
 //  - four lanes take an entry, an arc each, so its arcs are one address to
 //    the cache and its own word another; a lane holds one, two or four
 //    entries at a time (a lane with four arcs of one entry: 20% slower at 512
@@ -244,12 +250,13 @@ __device__ __forceinline__ void bin_near(NearQueues<NT> &q, int b, uint32_t n, i
 
 // This wave's new entries into queue b (near lanes) and at `far`: one LDS
 // atomic makes room for both (counters: near low, far high).  more: memory for
-// the near entries past the queue's room.
+// the near entries past the queue's room, or all of them (wide).
 template <int NT, int N>
 __device__ __forceinline__ void wave_put(NearQueues<NT> &q, int b, const bool (&near)[N],
                                          const bool (&farther)[N], const uint32_t (&v)[N],
                                          nf_range (&r)[N], unsigned long long *cnt,
-                                         uint32_t *rest, uint32_t *more, uint32_t *far) {
+                                         uint32_t *rest, bool wide, uint32_t *more,
+                                         uint32_t *far) {
   using Q = NearQueues<NT>;
   unsigned long long mn[N], mf[N];
   uint32_t tn = 0, tf = 0;
@@ -264,31 +271,26 @@ __device__ __forceinline__ void wave_put(NearQueues<NT> &q, int b, const bool (&
   unsigned long long base = 0;
   if (lane_prefix(~0ull) == 0) base = atomicAdd(cnt, ((unsigned long long)tf << 32) | tn);
   if (tn) {
+    uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base);
 #pragma unroll
     for (int k = 0; k < N; k++) {
-      const bool big = near[k] && r[k].y - r[k].x > 4;
+      const uint32_t x = at + lane_prefix(mn[k]);
+      const bool in = near[k] && !wide && x < Q::CAP;
+      const bool big = in && r[k].y - r[k].x > 4;
       const unsigned long long m = __ballot(big);
       if (m) {
-        uint32_t at = 0;
-        if (lane_prefix(~0ull) == 0) at = atomicAdd(rest, (uint32_t)__popcll(m));
-        at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) + lane_prefix(m);
-        if (big && at < Q::REST) {
-          q.rv[b][at] = v[k];
-          q.re[b][at] = (uint32_t)r[k].x + 4u;
-          q.rend[b][at] = (uint32_t)r[k].y;
+        uint32_t to = 0;
+        if (lane_prefix(~0ull) == 0) to = atomicAdd(rest, (uint32_t)__popcll(m));
+        to = (uint32_t)__builtin_amdgcn_readfirstlane((int)to) + lane_prefix(m);
+        if (big && to < Q::REST) {
+          q.rv[b][to] = v[k];
+          q.re[b][to] = (uint32_t)r[k].x + 4u;
+          q.rend[b][to] = (uint32_t)r[k].y;
           r[k].y = r[k].x + 4;
         }
       }
-    }
-    uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base);
-    const bool room = at + tn <= Q::CAP;
-#pragma unroll
-    for (int k = 0; k < N; k++) {
-      if (near[k]) {
-        const uint32_t x = at + lane_prefix(mn[k]);
-        if (room || x < Q::CAP) q.put(b, x, v[k], r[k]);
-        else more[x] = v[k];
-      }
+      if (in) q.put(b, x, v[k], r[k]);
+      else if (near[k]) more[x] = v[k];
       at += (uint32_t)__popcll(mn[k]);
     }
   }
@@ -334,7 +336,8 @@ __global__ __launch_bounds__(NT) void sssp_nf_kernel(
     for (int v = tid; v < V; v += NT) W[v] = v == src ? nf_word(0, 1u) : nf_word(FAP_INF, 0u);
     uint32_t *fa = q0 + 2 * (int64_t)V, *fb = q0 + 3 * (int64_t)V;
     int qb = 1;  // the queue that is filled; the other one is worked on
-    uint32_t n_near = 1, n_rest = 0, n_far = 0;
+    uint32_t *mw = q0, *mf = q0 + V;  // their entries in memory
+    uint32_t n_near = 1, n_lds = 1, n_rest = 0, n_far = 0;  // the first n_lds are in LDS
     if (tid == 0) s_q.put(0, 0, (uint32_t)src, range(src));
     uint32_t tags = 2;  // last tag handed out: 1 = the source's, 2 = the first far pile's
     uint32_t ft = 2;
@@ -349,18 +352,32 @@ __global__ __launch_bounds__(NT) void sssp_nf_kernel(
         s_rest[cz] = 0;
       }
     };
-    auto take = [&]() {
+    auto take = [&](bool wide) {
       const unsigned long long c = s_cnt[ci];
       const uint32_t nr = s_rest[ci];
       n_near = (uint32_t)c;
       n_rest = nr < Q::REST ? nr : Q::REST;
+      n_lds = wide ? 0 : n_near < Q::CAP ? n_near : Q::CAP;
       ci = ci == 2 ? 0 : ci + 1;
-      // entries past the LDS queue are in memory: everyone's stores first
-      if (n_near > Q::CAP) __syncthreads();
+      // entries in memory: everyone's stores first
+      if (n_near > n_lds) __syncthreads();
       qb ^= 1;
+      uint32_t *t = mw;
+      mw = mf;
+      mf = t;
       if constexpr (BIN) {
-        if (n_near >= bin_min && n_near <= Q::CAP)
+        if (n_near >= bin_min && n_near == n_lds) {
           bin_near<NT>(s_q, qb ^ 1, n_near, bsh, s_hist, s_wsum);
+        } else if (n_near >= bin_min) {
+          // (ranges are read again with the vertices, so the rest list goes)
+          for (uint32_t i = tid; i < n_lds; i += NT) mw[i] = s_q.v[qb ^ 1][i];
+          n_lds = n_rest = 0;
+          __syncthreads();
+          bin_queue<NT>(mw, mf, n_near, bsh, s_hist, s_wsum);
+          t = mw;
+          mw = mf;
+          mf = t;
+        }
       }
       return (uint32_t)(c >> 32);
     };
@@ -368,7 +385,7 @@ __global__ __launch_bounds__(NT) void sssp_nf_kernel(
       while (n_near > 0) {
         const uint32_t R = ++tags;
         const uint32_t n = n_near + n_rest;
-        const bool look = n >= NT / 8;
+        const bool look = n >= NT / 8, wide = n_near > Q::CAP;
         // four lanes to an entry, an arc each; a lane takes part in N entries,
         // NT / 4 apart
         auto relax = [&](auto width, uint32_t i0) {
@@ -381,12 +398,12 @@ __global__ __launch_bounds__(NT) void sssp_nf_kernel(
             u[k] = 0;
             e[k] = end[k] = 0;
             if (i < n_near) {
-              if (i < Q::CAP) {
+              if (i < n_lds) {
                 u[k] = s_q.v[qb ^ 1][i];
                 e[k] = (int)s_q.e[qb ^ 1][i];
                 end[k] = (int)s_q.end[qb ^ 1][i];
               } else {
-                u[k] = q0[(int64_t)(qb ^ 1) * V + i];
+                u[k] = mw[i];
                 const nf_range r = range(u[k]);
                 e[k] = r.x;
                 end[k] = r.y;
@@ -446,10 +463,9 @@ __global__ __launch_bounds__(NT) void sssp_nf_kernel(
             if (look) {
 #pragma unroll
               for (int k = 0; k < N; k++)
-                if (pn[k]) r[k] = range(v[k]);
+                if (pn[k] && !wide) r[k] = range(v[k]);
             }
-            wave_put<NT, N>(s_q, qb, pn, pf, v, r, &s_cnt[ci], &s_rest[ci], q0 + (int64_t)qb * V,
-                            fa + n_far);
+            wave_put<NT, N>(s_q, qb, pn, pf, v, r, &s_cnt[ci], &s_rest[ci], wide, mf, fa + n_far);
 #pragma unroll
             for (int k = 0; k < N; k++) e[k] += 4;
           }
@@ -468,7 +484,7 @@ __global__ __launch_bounds__(NT) void sssp_nf_kernel(
         }
         clear_next();
         lds_barrier();
-        n_far += take();
+        n_far += take(wide);
       }
       if (n_far == 0) break;
       // ---- threshold = min live far distance + delta ----
@@ -503,12 +519,12 @@ __global__ __launch_bounds__(NT) void sssp_nf_kernel(
             W[v[0]] = nf_word(d, pn[0] ? rs : fn);
           }
         }
-        wave_put<NT, 1>(s_q, qb, pn, pf, v, r, &s_cnt[ci], &s_rest[ci], q0 + (int64_t)qb * V, fb);
+        wave_put<NT, 1>(s_q, qb, pn, pf, v, r, &s_cnt[ci], &s_rest[ci], false, mf, fb);
       }
       ft = fn;
       clear_next();
       __syncthreads();
-      n_far = take();
+      n_far = take(false);
       uint32_t *t = fa;
       fa = fb;
       fb = t;

@@ -1,11 +1,11 @@
-// floyd.hip -- blocked Floyd-Warshall closure on the VALU, in place.
+// floyd.hip -- blocked Floyd-Warshall closure, in place.
 //
 // Replaces the reference's stage-2 operator floyd_path (fap/kernel/floyd.h:
 // 150-158; CPU semantics floyd_CPU_path :38-49: k-i-j order, strict relax).
 // The closure of a non-negative matrix is unique, so the blocked order gives
 // the same distances as the k-i-j loop.  With block size T (64 or 128) and
 // nb = ceil(n / T) blocks, round r (pivot block r) runs:
-//   1. diagonal tile (r, r): closed in one workgroup, in LDS;
+//   1. diagonal tile (r, r): closed in one workgroup, in registers;
 //   2. row panel (r, J) = min(C, D_rr (x) C) and column panel
 //      (I, r) = min(C, C (x) D_rr) for all I, J != r: one launch;
 //   3. every other tile (I, J) = min(C, D_Ir (x) D_rJ): one launch.
@@ -370,14 +370,9 @@ static int run_rounds(int32_t *d, int32_t n, int64_t ld, hipStream_t s) {
 }
 
 // Block size and look-ahead: the context options if set, else the tune
-// cache, else 128 when phase 3 has at least 4 tiles of 128 per CU and 64
-// below, without look-ahead (fw_settings).  Measured on MI355X (closure
-// ms, T = 64 / 128): n = 8192 20.7 / 19.0, 6144 9.49 / 8.86, 5120 5.99 /
-// 6.54, 4096 3.59 / 4.87, 2048 1.40 / 1.83 -- the 128 x 128 tile with 8 x 8
-// cells per lane halves the LDS bytes per update of the 64 x 64 tile's
-// 4 x 4 cells, and with the next diagonal closed inside phase 3 and the
-// panels split in quarters, the serial phases of T = 128 no longer cost
-// more than that saves once the grid is large.
+// cache, else 128 for large n and 64 below, without look-ahead (fw_settings,
+// with both sides measured).  T = 128 halves the passes over the matrix, but
+// its chain of diagonal and panels is longer.
 int launch_fw(fap_ctx *ctx, int32_t *d, int32_t n, int64_t ld, hipStream_t s) {
   if (n <= 0) return FAP_OK;
   int tile;

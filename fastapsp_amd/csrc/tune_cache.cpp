@@ -75,12 +75,15 @@ fap_tune_cache *tune_env_cache() {
 void fw_settings(const fap_ctx *ctx, int32_t n, int *tile, bool *lookahead) {
   int32_t p[2] = {64, 0};
   const bool cached = tune_lookup(ctx, "fw", fap_tune_key_fw(n), p);
-  // default: 128 once phase 3 has at least 4 tiles of 128 x 128 per CU (n >=
-  // 4225 on 256 CUs), where it measured faster (4096: 3.67 ms, 3.37 at 64;
-  // 4500: 4.20 and 4.69); 64 below
+  // default: 128 once phase 3 has at least 4.5 tiles of 128 x 128 per CU (n >=
+  // 4353 on 256 CUs), 64 below.  Measured, ms at 64 / 128, distances below 2^22
+  // and then beyond them (integer additions): 3840 2.62 / 3.47, 3.19 / 3.64; 4200
+  // 3.36 / 3.91, 4.24 / 4.14; 4352 3.52 / 4.00, 4.36 / 4.21; 4500 4.00 / 4.24,
+  // 5.16 / 4.60; 5120 5.26 / 5.03, 6.74 / 6.13; 5500 6.58 / 5.77, 8.53 / 7.66.
+  // Between 4353 and 4800 the line favours the second kind: 6% there against 12.
   const int64_t nb128 = ((int64_t)n + 127) / 128;
   const int def_tile =
-      (nb128 - 1) * (nb128 - 1) >= 4 * (int64_t)(ctx ? ctx->num_cus : 256) ? 128 : 64;
+      2 * (nb128 - 1) * (nb128 - 1) >= 9 * (int64_t)(ctx ? ctx->num_cus : 256) ? 128 : 64;
   *tile = (ctx && (ctx->opt_fw_tile == 64 || ctx->opt_fw_tile == 128)) ? ctx->opt_fw_tile
           : cached                                                     ? p[0]
                                                                        : def_tile;

@@ -19,7 +19,7 @@
  *   "batch"  fap_tune_key_batch(count, n)          {workgroups per CU per launch}
  *
  * With no entry the defaults are tile 128 when ceil(n / 128) - 1 squared is
- * at least 4 per CU (64 below), no look-ahead, SSSP threads 1024
+ * at least 4.5 per CU (64 below), no look-ahead, SSSP threads 1024
  * while the sources fit on the CUs (512 up to twice that, beyond it 256, or 512 from
  * 2^17 vertices),
  * delta 8 x mean weight while the sources fit on the CUs (6 x up to twice

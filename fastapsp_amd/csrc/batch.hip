@@ -286,7 +286,7 @@ __global__ void fw_queue_reset_kernel(int32_t *ctrl, int nctrl, int32_t *done, i
 
 namespace fapi {
 
-constexpr int64_t kPair128MinTiles = 2 * 256;  // two per CU of an MI355X
+constexpr int64_t kPair128MinTiles = 2 * 256;  // two per CU of an MI355X (no context here)
 
 // Launch p of a batch holds phase p of every job that has one, jobs in
 // decreasing size (longest processing time first), each job's phase one

@@ -148,7 +148,6 @@ struct DenseJob {
   const int2 *edges;
   int32_t *mat;
   int64_t ld;
-  int64_t cell_base;  // prefix of n^2 over earlier jobs
   int32_t row_base;   // prefix of n over earlier jobs
   int32_t n;
 };
@@ -236,7 +235,7 @@ int fw_plan_run(fap_fw_plan *p, hipStream_t s);
 void fw_plan_destroy(fap_fw_plan *p);
 
 // Dense build of jobs already on the device; `cells` = sum n^2, `rows` = sum n.
-int launch_dense_jobs(fap_ctx *ctx, const fapk::DenseJob *d_jobs, int32_t njobs, int64_t cells,
-                      int64_t rows, hipStream_t s);
+int launch_dense_jobs(fap_ctx *ctx, const fapk::DenseJob *d_jobs, int32_t njobs, int64_t rows,
+                      hipStream_t s);
 
 }  // namespace fapi

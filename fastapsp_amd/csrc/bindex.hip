@@ -93,8 +93,9 @@ struct BidxTile {
 // Control words of the block iterations (device).
 enum { BC_THR = 0, BC_NTILES = 2, BC_DONE = 3, BC_WORDS = 16 };
 
-// Longest border-position list a tile may take (the sum of a part's
-// in-border lengths); a graph with a longer one gets no index.
+// Longest border-position list (the sum of a part's in-border lengths); a graph
+// with a longer one gets no index.  Its block updates would take many pieces of
+// kListSeg and were never measured against SSSP rows.
 constexpr int kBidxKlMax = 2048;
 
 // Expansion tiles: 16 kExpandTM sources x kExpandCols columns of a part.
@@ -932,7 +933,7 @@ int bidx_build(fap_ctx *ctx, fap_graph_dev *g) {
       }
       inb_off[q2 + 1] = inb_off[q2] + slot;
       const int32_t kl = inb_pos_off.back() - inb_pos_off[inb_off[q2]];
-      if (kl > kBidxKlMax) {  // a tile's border list would not fit in LDS
+      if (kl > kBidxKlMax) {
         delete x;
         return FAP_OK;
       }

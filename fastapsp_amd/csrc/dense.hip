@@ -89,9 +89,9 @@ __global__ __launch_bounds__(64 * DR_WAVES) void dense_rows_kernel(const DenseJo
 
 namespace fapi {
 
-int launch_dense_jobs(fap_ctx *ctx, const fapk::DenseJob *d_jobs, int32_t njobs, int64_t cells,
-                      int64_t rows, hipStream_t s) {
-  if (njobs <= 0 || cells <= 0) return FAP_OK;
+int launch_dense_jobs(fap_ctx *ctx, const fapk::DenseJob *d_jobs, int32_t njobs, int64_t rows,
+                      hipStream_t s) {
+  if (njobs <= 0 || rows <= 0) return FAP_OK;
   if (rows > INT32_MAX) return fail(FAP_E_ARG, "dense build: too many rows");
   const int64_t blocks = std::min<int64_t>((rows + fapk::DR_WAVES - 1) / fapk::DR_WAVES,
                                            (int64_t)ctx->num_cus * 32);
@@ -105,14 +105,11 @@ int run_dense_from_graphs(fap_ctx *ctx, int32_t count, const fap_graph_dev *cons
                           int32_t *const *mats, const int64_t *ld, hipStream_t s) {
   std::vector<fapk::DenseJob> jobs;
   jobs.reserve(count);
-  int64_t cells = 0;
   int64_t rows = 0;
   for (int32_t j = 0; j < count; j++) {
     const fap_graph_dev *g = graphs[j];
     if (g->V == 0) continue;
-    jobs.push_back(fapk::DenseJob{g->row_offset, g->edges, mats[j], ld[j], cells, (int32_t)rows,
-                                  g->V});
-    cells += (int64_t)g->V * g->V;
+    jobs.push_back(fapk::DenseJob{g->row_offset, g->edges, mats[j], ld[j], (int32_t)rows, g->V});
     rows += g->V;
   }
   if (jobs.empty()) return FAP_OK;
@@ -121,7 +118,7 @@ int run_dense_from_graphs(fap_ctx *ctx, int32_t count, const fap_graph_dev *cons
   FAP_TRY(ensure_ws(ctx, ctx->ws_dense, bytes));
   FAP_HIP(hipMemcpyAsync(ctx->ws_dense.ptr, jobs.data(), bytes, hipMemcpyHostToDevice, s));
   FAP_TRY(launch_dense_jobs(ctx, (const fapk::DenseJob *)ctx->ws_dense.ptr, (int32_t)jobs.size(),
-                            cells, rows, s));
+                            rows, s));
   // the descriptor copy reads `jobs` asynchronously
   FAP_HIP(hipStreamSynchronize(s));
   return FAP_OK;

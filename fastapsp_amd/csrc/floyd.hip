@@ -148,7 +148,6 @@ __global__ __launch_bounds__(FW_DIAG_THREADS) void fw_round_kernel(int32_t *d, i
 // aliases one operand; the tile reads all operands before writing C.  On the
 // matrix-core tile, as phase 3, for any alignment (n = 2999 at an odd row
 // stride 2.95 -> 2.01 ms with both; the 4 x 4 integer tile before).
-template <int TM>
 __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6))) void fw_panel_kernel(
     int32_t *d, int n, int64_t ld, int r, int nb, int flags) {
   using Tile = MxSmall;
@@ -299,8 +298,8 @@ struct Fw {
         hipLaunchKernelGGL(fapk::fw_panel128_kernel, dim3(8 * (nb - 1)), dim3(fapk::MP_THREADS),
                            0, s, d, n, ld, r, nb, flags);
       else
-        hipLaunchKernelGGL(fapk::fw_panel_kernel<TM>, dim3(2 * (nb - 1)),
-                           dim3(fapk::MP_THREADS), 0, s, d, n, ld, r, nb, flags);
+        hipLaunchKernelGGL(fapk::fw_panel_kernel, dim3(2 * (nb - 1)), dim3(fapk::MP_THREADS), 0, s,
+                           d, n, ld, r, nb, flags);
       FAP_CHECK_LAUNCH();
     }
     return FAP_OK;

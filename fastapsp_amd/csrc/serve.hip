@@ -402,19 +402,17 @@ int launch_wave(fap_server *S, Lane &L) {
       lds[j] = r->ld;
     }
     std::vector<fapk::DenseJob> dj;
-    int64_t cells = 0, rows = 0;
+    int64_t rows = 0;
     for (int32_t j = 0; j < cnt; j++) {
       dj.push_back(fapk::DenseJob{(const int32_t *)(L.d_stage + o_ro[j]),
-                                  (const int2 *)(L.d_stage + o_e[j]), mats[j], lds[j], cells,
+                                  (const int2 *)(L.d_stage + o_e[j]), mats[j], lds[j],
                                   (int32_t)rows, ns[j]});
-      cells += (int64_t)ns[j] * ns[j];
       rows += ns[j];
     }
     // Graphs of at least DENSE_PATH_N vertices are closed one by one with
-    // the dense blocked FW (one such closure fills the GPU, and its fused
-    // diagonal and single-kind launches close n = 4096 in 3.5 ms against
-    // 6.1 ms in the batched closure); smaller ones share one batched
-    // closure, where they run side by side.
+    // the dense blocked FW, smaller ones share one batched closure, where they
+    // run side by side (n = 4096: one alone 3.07 ms, 4.10 in the batched
+    // closure; three 9.16 and 7.54).
     std::vector<int32_t *> bmats;
     std::vector<int32_t> bns;
     std::vector<int64_t> blds;
@@ -437,8 +435,7 @@ int launch_wave(fap_server *S, Lane &L) {
     const size_t o_sg = put(fd.segs.data(), sizeof(fapk::BatchSeg) * fd.segs.size());
     if (off > (size_t)S->opts.stage_bytes) return fail(FAP_E_NOMEM, "wave staging overflow");
     FAP_HIP(hipMemcpyAsync(L.d_stage, h, off, hipMemcpyHostToDevice, s));
-    FAP_TRY(launch_dense_jobs(L.ctx, (const fapk::DenseJob *)(L.d_stage + o_dj), cnt, cells, rows,
-                              s));
+    FAP_TRY(launch_dense_jobs(L.ctx, (const fapk::DenseJob *)(L.d_stage + o_dj), cnt, rows, s));
     // With both kinds in the wave, the big graphs run on the lane
     // context's auxiliary stream beside the batched closure of the small
     // ones; the wave's completion (recorded on s) waits for both.

@@ -70,7 +70,7 @@ int fap_ctx_stream(fap_ctx *ctx, void **stream);
  * fw_lookahead; the defaults) defers to the context's tune cache
  * (fap_tune.h), then to the default in brackets:
  *   "fw_lookahead" -1/0/1   overlap FW round r+1's diagonal/panels with round r [0]
- *   "fw_tile"      0/64/128 FW block size [64]
+ *   "fw_tile"      0/64/128 FW block size [128 from 4,353 vertices on 256 CUs, else 64]
  *   "sssp_threads" 0/256/512/1024  threads per SSSP workgroup [1024 while the sources
  *                           fit on the CUs, 512 up to twice that, beyond that 256, or
  *                           512 for graphs of 2^17 vertices and more]

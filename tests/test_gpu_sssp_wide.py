@@ -49,3 +49,23 @@ def test_wide_fronts(gpu_ctx, graph, threads, binq):
     d_src.free()
     out.free()
     dg.close()
+
+
+# beyond two sources a compute unit: 256 threads a source, or 512 from 2^17 vertices on
+@pytest.mark.parametrize("side", [362, 363])
+def test_threads_by_vertex_count(gpu_ctx, side):
+    from fastapsp_amd import synth
+    V = side * side
+    u, v, w = synth.grid_graph(side, side, 0.10, 0.02, 1, 100, 3)
+    ro, col, w = synth.to_csr(V, u, v, w, False)
+    src = np.random.default_rng(side).choice(V, 513, replace=False).astype(np.int32)
+    dg = gpu_ctx.upload_graph(ro, col, w)
+    d_src, out = gpu_ctx.to_device(src), gpu_ctx.alloc((src.size, V))
+    dg.sssp(d_src.ptr, src.size, out.ptr, V)
+    gpu_ctx.sync()
+    got = out.get()
+    at = [0, 1, 255, 256, 511, 512]
+    np.testing.assert_array_equal(got[at], O.batched_sssp(src[at], ro, col, w))
+    d_src.free()
+    out.free()
+    dg.close()

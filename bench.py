@@ -63,13 +63,13 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 VALU_PEAK_TOPS = 256 * 64 * 2.4e9 / 1e12  # spec: 1 int32 op per lane per clock, 39.32 T
-MX_MIX_TOPS = 102.0  # MFMA outer sums and v_min3_i32, 4 waves per SIMD
+MX_MIX_TOPS = 104.0  # MFMA outer sums and v_min3_i32, 4 waves per SIMD (102.0 and 104.1 in two runs)
 # HBM bytes per launch of the n = 8192 min-plus product and per n = 8192
 # tile-128 FW closure, from two rocprofv3 counter runs (FETCH_SIZE x 2.0 +
-# WRITE_SIZE x 1.0, scales from a copy of known size): product 6.47e9 read
-# + 0.27e9 written; closure 34.07e9 read + 17.44e9 written.
-MINPLUS_8192_TRAFFIC = 6.74e9
-FW_8192_T128_TRAFFIC = 51.51e9
+# WRITE_SIZE x 1.0, scales from a copy of known size): product 7.65e9 read
+# + 0.27e9 written; closure 34.88e9 read + 18.86e9 written.
+MINPLUS_8192_TRAFFIC = 7.92e9
+FW_8192_T128_TRAFFIC = 53.74e9
 HBM_PEAK_GBS = 8000.0
 
 

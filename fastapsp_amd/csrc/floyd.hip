@@ -218,7 +218,7 @@ __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(8)))
 // swapping with the workgroup that had it -- and after its update closes
 // it (in LDS for T = 64, by close_block128 for T = 128): the next round's
 // diagonal phase, done while the other tiles of this phase run, so that
-// round launches only its panels.  T = 64 wants 6 waves per SIMD (77 VGPRs, no
+// round launches only its panels.  T = 64 wants 6 waves per SIMD (78 to 80 VGPRs, no
 // call inside): n = 3500 2.58 ms, 2.73 at the 4 that its callees would leave.
 template <int TM, bool fuse>
 __global__ __launch_bounds__(MP_THREADS) __attribute__((amdgpu_waves_per_eu(TM == 4 ? 6 : 4, TM == 4 ? 6 : 4))) void fw_rest_kernel(

@@ -29,11 +29,11 @@
 // look costs products of few k (4096 x 65536 x 16 241 -> 272 us).
 //
 // What bounds it: the VALU port, 16 v_min3_i32 and one MFMA issue for 2048
-// sums.  Measured in registers and LDS alone (4 waves per SIMD): 102 TOP/s at
+// sums.  Measured in registers and LDS alone (4 waves per SIMD): 104 TOP/s at
 // 2 ops per update against 70.3 of add, add, min3 (MFMA alone 149, v_min3
 // alone 137; the clock falls to 2.1 GHz with both units busy).  Kernels on the
 // 128 x 128 tile, integer tile before: the 8192^3 product 16.4 -> 10.8 ms
-// (102 TOP/s), 909 x 262144 x 115 0.936 -> 0.68 ms, the n = 8192 closure
+// (102 TOP/s), 909 x 262144 x 115 0.936 -> 0.66 ms, the n = 8192 closure
 // 18.9 -> 15.1 ms.  It takes every 128-row tile of a product of 16 k and more
 // (row tails are in minplus.hip).
 #ifndef FAP_MFMA_TILE_H_
